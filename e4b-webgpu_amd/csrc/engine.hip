@@ -242,15 +242,16 @@ int expect(const char* name, int type, int want_type, const int64_t* dims, int n
 
 int record_step(e4b_ctx* c);
 
-// batched prefill: tokens per chunk at most, and split-K slices of the
-// o and down projection GEMMs (their consumers sum the slices)
+// batched prefill: tokens per chunk at most, and the most split-K slices of
+// the projection GEMMs (their consumers sum them; a chunk's number is
+// q40_gemm_best_kslices)
 constexpr int kPfMaxChunk = 512;
-constexpr int kPfKsO = 4;    // o projection
-constexpr int kPfKs = 8;     // down projection (the most slices; sizes the partial buffer)
-constexpr int kPfKsQkv = 2;  // qkv (the head prep sums the slices)
-constexpr int kPfKsPle = 8;  // PLE gate (256 rows; the GELU-multiply kernel sums the slices)
-constexpr int kPfA4bOKs = 4;
-constexpr int kPfA4bQkvKs = 2;  // A4B q|k|v projection (the head prep sums the slices)  // A4B o projection (the attention-residual row norm sums the slices)
+constexpr int kPfKsO = 4;       // o projection (the residual row norm sums the slices)
+constexpr int kPfKs = 8;        // down projection (the most slices; sizes the partial buffer)
+constexpr int kPfKsQkv = 2;     // qkv (the head prep sums the slices)
+constexpr int kPfKsPle = 8;     // PLE gate (the GELU-multiply kernel sums the slices)
+constexpr int kPfA4bOKs = 4;    // A4B o projection (the attention-residual row norm)
+constexpr int kPfA4bQkvKs = 2;  // A4B q|k|v projection (the head prep)
 
 }  // namespace
 
@@ -1080,7 +1081,7 @@ int prefill_chunk_a4b(e4b_ctx* c, uint32_t p0, int M) {
   const int64_t MH = (int64_t)M * H;
   hipStream_t st = c->st;
   int rc;
-  auto gemm = [&](const Q40Mat& W, const uint16_t* X, int ldx, float* Y, int ks_want = 1) {
+  auto gemm = [&](const Q40Mat& W, const uint16_t* X, int ldx, float* Y, int ks) {
     GemmArgs g{};
     g.W = W;
     g.X = X;
@@ -1088,12 +1089,9 @@ int prefill_chunk_a4b(e4b_ctx* c, uint32_t p0, int M) {
     g.ldx = ldx;
     g.epi = GEMM_F32;
     g.Y = Y;
-    g.ks = q40_gemm_kslices(W.nb, ks_want);
+    g.ks = ks;
     return launch_q40_gemm(g, st);
   };
-  // the o projection's K slices (its 2816 output rows alone give too few
-  // workgroups): what q40_gemm_kslices makes of kPfA4bOKs for the layer
-  auto ok_slices = [&](const Layer& ly) { return q40_gemm_kslices(QH * ly.hd / 32, kPfA4bOKs); };
   const Q6Mat E = q6_view(c->embd, k.vocab, H);
   if ((rc = launch_embed_rows(E, c->pf_ids, M, sqrtf((float)H), c->pf_h, c->pf_xhl, st)) ||
       (rc = tick(c, "embed_rows")))
@@ -1101,10 +1099,12 @@ int prefill_chunk_a4b(e4b_ctx* c, uint32_t p0, int M) {
   for (int l = 0; l < Lc; ++l) {
     const Layer& ly = c->L[l];
     const int window = ly.global ? 0 : k.window;
+    const int ks_qkv = q40_gemm_best_kslices(ly.qkv_rows, H / 32, M, kPfA4bQkvKs);
+    const int ks_o = q40_gemm_best_kslices(H, QH * ly.hd / 32, M, kPfA4bOKs);
     if ((rc = launch_rownorm(c->pf_h, nullptr, nullptr, nullptr, 1.f, ly.attn_norm, c->pf_xn, nullptr, H, k.eps, st,
                              M)) ||
         (rc = tick(c, "norm_rows")) ||
-        (rc = gemm(q40_view(ly.qkv, ly.qkv_rows, H), c->pf_xn, H, c->pf_qkv, kPfA4bQkvKs)) ||
+        (rc = gemm(q40_view(ly.qkv, ly.qkv_rows, H), c->pf_xn, H, c->pf_qkv, ks_qkv)) ||
         (rc = tick(c, "gemm_qkv")))
       return rc;
     HeadRowsGen hr{};
@@ -1125,7 +1125,7 @@ int prefill_chunk_a4b(e4b_ctx* c, uint32_t p0, int M) {
     hr.keqv = ly.keqv;
     hr.p0 = p0;
     hr.eps = k.eps;
-    hr.ks = q40_gemm_kslices(H / 32, kPfA4bQkvKs);
+    hr.ks = ks_qkv;
     hr.slice = (int64_t)M * ly.qkv_rows;
     // the matrix-core attention of the prefill (split keys + combine); other
     // head shapes: one workgroup per (KV group, token)
@@ -1158,11 +1158,11 @@ int prefill_chunk_a4b(e4b_ctx* c, uint32_t p0, int M) {
     if ((rc = launch_headprep_rows_gen(hr, M, st)) || (rc = tick(c, "headprep_rows")) ||
         (rc = mfma_attn ? launch_attn_prefill(pa, st) : launch_attn_rows_gen(ar, M, st)) ||
         (rc = tick(c, "attn_rows")) ||
-        (rc = gemm(q40_view(ly.o, H, (int64_t)QH * ly.hd), c->pf_attn, QH * ly.hd, c->pf_y, kPfA4bOKs)) ||
+        (rc = gemm(q40_view(ly.o, H, (int64_t)QH * ly.hd), c->pf_attn, QH * ly.hd, c->pf_y, ks_o)) ||
         (rc = tick(c, "gemm_o")) ||
         // h1 = h + rms(o) post_attn, in place (o: the sum of the K slices)
         (rc = launch_rownorm(c->pf_h, c->pf_h, c->pf_y, ly.post_attn, 1.f, nullptr, nullptr, nullptr, H, k.eps, st,
-                             M, ok_slices(ly), MH)) ||
+                             M, ks_o, MH)) ||
         (rc = tick(c, "attn_residual_rows")))
       return rc;
     MoeArgs a = c->moe;
@@ -1250,8 +1250,10 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
                                 k.eps, st)) ||
       (rc = tick(c, "resnorm_rows")))
     return rc;
-  const int ks_o = q40_gemm_kslices(QH * HD / 32, kPfKsO), ks_d = q40_gemm_kslices(FF / 32, kPfKs);
-  const int ks_qkv = q40_gemm_kslices(H / 32, kPfKsQkv), ks_pg = q40_gemm_kslices(H / 32, kPfKsPle);
+  const int ks_o = q40_gemm_best_kslices(H, QH * HD / 32, M, kPfKsO);
+  const int ks_d = q40_gemm_best_kslices(H, FF / 32, M, kPfKs);
+  const int ks_qkv = q40_gemm_best_kslices(c->qkv_rows, H / 32, M, kPfKsQkv);
+  const int ks_pg = q40_gemm_best_kslices(PD, H / 32, M, kPfKsPle);
   for (int l = 0; l < Lc; ++l) {
     const Layer& ly = c->L[l];
     // attention block

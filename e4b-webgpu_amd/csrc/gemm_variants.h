@@ -1,0 +1,17 @@
+// gemm_variants.h -- the q4_0 GEMM variants, by translation unit.
+#pragma once
+#include "gemm_kernel.h"
+
+namespace gemm {
+struct VariantSet {
+  const Variant* v;
+  int n;
+};
+VariantSet variants_f32();      // rows of an even number of blocks
+VariantSet variants_glu();
+VariantSet variants_mul();
+VariantSet variants_f32_odd();  // of an odd number
+VariantSet variants_glu_odd();
+VariantSet variants_mul_odd();
+VariantSet variants_grp(bool glu, bool aligned);  // grouped: one each
+}  // namespace gemm

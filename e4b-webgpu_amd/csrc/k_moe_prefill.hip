@@ -6,10 +6,10 @@
 //
 //   router + top-8      the decode kernels over token rows (bit-identical picks)
 //   k_moe_group         counting sort of the M*8 (token, slot) draws by expert
-//                       into contiguous runs, cut into tiles of <= 32 rows
+//                       into contiguous runs, cut into tiles of <= 64 rows
 //   grouped GEMMs       expert gate/up + GeGLU and expert down on the matrix
 //                       cores (k_gemm.hip grouped mode): each tile reads its
-//                       expert's rows once for up to 32 draws
+//                       expert's rows once for up to 64 draws
 //   dense branch        gate|up GEMM in K slices, k_geglu_rows, down GEMM in
 //                       K slices over all M tokens
 //   k_moe_combine_rows  moe[m] = sum_k w_k down_sorted[pos(m, k)], in k order,
@@ -23,7 +23,7 @@
 namespace {
 
 constexpr int K = kMoeTopK;
-constexpr int kTileRows = 32;
+constexpr int kTileRows = 64;  // the grouped GEMM's row tile
 
 // one workgroup: histogram of the draws' experts in LDS, exclusive scan,
 // placement (list[slot] = draw, pos[draw] = slot) and the tile table.  The

@@ -133,7 +133,7 @@ struct GemmArgs {
   int64_t mul_ld;
   int ks;             // split-K slices (GEMM_F32)
   // grouped mode (the expert-indexed MoE prefill; tiles != null): blockIdx.y
-  // picks tiles[y] = (group g, first row r0, rows n <= 32) of the M sorted
+  // picks tiles[y] = (group g, first row r0, rows n <= 64) of the M sorted
   // rows, y < *ntiles; the weights are rows [g group_rows, (g+1) group_rows)
   // of W (GLU: group_rows = 2 ff, gate then up); X row r is gather[r] /
   // gather_div (gather null: row r); outputs are rows r0 .. r0 + n - 1 of an
@@ -149,6 +149,9 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st);
 // the largest split-K slice count <= want that cuts nb blocks into whole
 // slices (what GemmArgs::ks must be)
 int q40_gemm_kslices(int nb, int want);
+// the slice count <= most that makes an f32 product of M tokens and its
+// consumer's sum over the slices fastest
+int q40_gemm_best_kslices(int64_t rows, int nb, int M, int most);
 int launch_q40(const Q40Mat& W, const uint32_t* xh, const uint32_t* xl, int epi, const GemvOut& o, int ks,
                hipStream_t st, const ProArgs* pro = nullptr);
 int launch_q40_gemv(const Q40Mat& W, const uint32_t* xh, const uint32_t* xl, float* y, hipStream_t st);

@@ -248,7 +248,7 @@ int e4b_k_moe_layer(const e4b_moe_weights* w, const float* h, float* h_out, uint
  * guGsg32 / downGsg32 + waccB, kernels/expgroup.wgsl:15-50,
  * kernels/q40gugrp.wgsl:47-103): per token the e4b_k_moe_layer arithmetic;
  * the m*8 expert draws are sorted by expert and each expert's weight rows
- * are read once per tile of up to 32 draws (MFMA GEMMs).  h, h_out
+ * are read once per tile of up to 64 draws (MFMA GEMMs).  h, h_out
  * f32[m][hidden]; topk_idx u32[m][8], topk_w f32[m][8], dense_out /
  * moe_out f32[m][hidden] may be NULL.  1 <= m <= 1024. */
 int e4b_k_moe_prefill(const e4b_moe_weights* w, const float* h, int m, float* h_out, uint32_t* topk_idx,

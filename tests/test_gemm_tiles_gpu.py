@@ -1,0 +1,96 @@
+"""GPU parity of every tile variant of the batched q4_0 GEMM, at the edges of
+its tiles, against float64 products of the same f16 activations and the
+oracle's dequantised weights.
+
+The variant follows from the shape (rows, columns, tokens); the first lists
+hold one shape for each, all ragged in rows and tokens and with a last K stage
+that is not full.  Products are exact and sums are f32, so outputs lie within
+1e-5 of max|Y| (2048 columns: f32 rounding of partial sums, 64 blocks x 2^-24,
+is 4e-6 at worst); the GeGLU adds one f16 rounding (2^-11) of the output.
+"""
+import numpy as np
+import pytest
+
+import oracle as orc
+from e4b import formats
+from e4b.kernels import MoeLayer, Q40Matrix
+from tests.util import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _dense(w, rows, cols):
+    return orc.q40_dequant(w).astype(np.float64).reshape(rows, cols)
+
+
+def _gelu(g):
+    return 0.5 * g * (1 + np.tanh(np.clip(0.7978845608028654 * (g + 0.044715 * g ** 3), -20, 20)))
+
+
+# rows of an even number of blocks (64 x 3 .. 2048), then of an odd number
+F32 = [(9176, 192, 639), (14280, 704, 217), (8591, 2048, 35), (14338, 384, 161), (102, 192, 3), (17554, 384, 1),
+       (61, 384, 5), (5306, 224, 689), (5696, 2016, 65), (151, 224, 2), (312, 288, 1), (33, 64, 33), (1, 32, 1)]
+GLU = [(6717, 192, 326), (6946, 192, 165), (6714, 192, 105), (6569, 384, 97), (76, 192, 2), (152, 384, 1),
+       (8744, 224, 139), (6557, 224, 100), (19, 224, 8), (33, 64, 33)]
+
+
+@pytest.mark.parametrize("rows,cols,m", F32)
+def test_f32_tiles(rows, cols, m):
+    w = formats.synth_q40(rows + cols + m, rows, cols, 0.02)
+    x = formats.synth_normal(rows + m, m * cols).reshape(m, cols).astype(np.float16)
+    got = Q40Matrix(w, rows, cols).gemm(x)
+    assert max_rel_err(got, x.astype(np.float64) @ _dense(w, rows, cols).T) < 1e-5
+
+
+@pytest.mark.parametrize("ff,cols,m", GLU)
+def test_geglu_tiles(ff, cols, m):
+    w = formats.synth_q40(ff + cols + m, 2 * ff, cols, 0.02)
+    x = formats.synth_normal(ff + m, m * cols).reshape(m, cols).astype(np.float16)
+    got = Q40Matrix(w, 2 * ff, cols).gemm_geglu(x).astype(np.float64)
+    y = x.astype(np.float64) @ _dense(w, 2 * ff, cols).T
+    want = _gelu(y[:, :ff]) * y[:, ff:]
+    assert np.max(np.abs(got - want) - (2.0 ** -11 * np.abs(want) + 1e-5 * np.abs(want).max())) <= 0
+
+
+def test_non_finite_token_stays_in_its_row():
+    # the last K stage of 7 blocks is completed with zeros, not with another
+    # block's activations: an infinity there reaches its own token only, and
+    # as the sum it is (weights of one sign: +inf, not NaN)
+    rows, cols, m = 70, 224, 40
+    w = formats.synth_q40(5, rows, cols, 0.02).reshape(-1, 18)
+    w[:, 2:] = (w[:, 2:] & 0x77) | 0x88
+    w[:, 2:] |= 0x11  # nibbles 9..15: every weight positive
+    x = formats.synth_normal(6, m * cols).reshape(m, cols).astype(np.float16)
+    x[17, cols - 1] = np.inf
+    got = Q40Matrix(w.reshape(-1), rows, cols).gemm(x)
+    assert np.all(got[17] == np.inf)
+    x[17, cols - 1] = 0
+    rest = np.delete(np.arange(m), 17)
+    ref = x.astype(np.float64) @ _dense(w.reshape(-1), rows, cols).T
+    assert max_rel_err(got[rest], ref[rest]) < 1e-5
+
+
+@pytest.mark.parametrize("m", [31, 65, 130, 300])
+def test_grouped_tiles(m):
+    # 9 experts, top 8: nearly every token reaches every expert, so a run of
+    # draws is cut into tiles of 64 with a remainder above and below 32 rows;
+    # expert FFN 96 = 3 blocks (odd), dense FFN 160
+    H, E, FF, FF2 = 512, 9, 96, 160
+    rng = np.random.default_rng(m)
+    q = lambda r, c, s: formats.synth_q40(s, r, c, 0.02)  # noqa: E731
+    vec = lambda: (1 + 0.1 * rng.standard_normal(H)).astype(np.float32)  # noqa: E731
+    t = {"ffn_norm": vec(), "router_scale": vec(), "pre_ffw2": vec(), "post_ffw1": vec(), "post_ffw2": vec(),
+         "post_ffw": vec(), "pes": (1 + 0.2 * rng.standard_normal(E)).astype(np.float32),
+         "router_w": formats.synth_normal(3, E * H, 0.0, 0.02).reshape(E, H), "dense_gate": q(FF2, H, 1),
+         "dense_up": q(FF2, H, 2), "dense_down": q(H, FF2, 3), "exp_gate_up": q(E * 2 * FF, H, 4),
+         "exp_down": q(E * H, FF, 5)}
+    h = formats.synth_normal(m, m * H).reshape(m, H)
+    got = MoeLayer(H, E, FF, FF2, t).prefill(h)
+    ref = dict(t, hidden=H, n_experts=E, top_k=8, expert_ffn=FF, dense_ffn=FF2)
+    for i in sorted({0, 1, m // 2, m - 2, m - 1}):
+        idx, wts, dense, moe, hout = orc.moe_ffn(ref, h[i])
+        np.testing.assert_array_equal(got["topk_idx"][i], idx)
+        # f16 branch inputs and GeGLU outputs, as the half-layer stores them
+        assert max_rel_err(got["dense_out"][i], dense) < 2e-3
+        assert max_rel_err(got["moe_out"][i], moe) < 2e-3
+        assert max_rel_err(got["h_out"][i], hout) < 1e-3
