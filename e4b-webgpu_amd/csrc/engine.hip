@@ -1212,8 +1212,7 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
   const int64_t MH = (int64_t)M * H;
   hipStream_t st = c->st;
   int rc;
-  auto gemm = [&](const Q40Mat& W, const uint16_t* X, int ldx, int epi, float* Y, uint16_t* Yh, int64_t ff,
-                  const float* mul, int64_t mul_ld, int ks) {
+  auto gemm = [&](const Q40Mat& W, const uint16_t* X, int ldx, int epi, float* Y, uint16_t* Yh, int64_t ff, int ks) {
     GemmArgs g{};
     g.W = W;
     g.X = X;
@@ -1223,8 +1222,6 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
     g.Y = Y;
     g.Yh = Yh;
     g.ff = ff;
-    g.mul = mul;
-    g.mul_ld = mul_ld;
     g.ks = ks;
     return launch_q40_gemm(g, st);
   };
@@ -1236,9 +1233,9 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
     // PLE model projection of the f32 embedding as two f16 GEMMs (hi, lo)
     const Q40Mat Wpm = q40_view(c->ple_proj, NP, H);
     const int64_t slice = (int64_t)M * NP;
-    if ((rc = gemm(Wpm, c->pf_xhl, H, GEMM_F32, c->pf_proj, nullptr, 0, nullptr, 0, 1)) ||
+    if ((rc = gemm(Wpm, c->pf_xhl, H, GEMM_F32, c->pf_proj, nullptr, 0, 1)) ||
         (rc = tick(c, "gemm_ple_model_proj")) ||
-        (rc = gemm(Wpm, c->pf_xhl + MH, H, GEMM_F32, c->pf_proj + slice, nullptr, 0, nullptr, 0, 1)) ||
+        (rc = gemm(Wpm, c->pf_xhl + MH, H, GEMM_F32, c->pf_proj + slice, nullptr, 0, 1)) ||
         (rc = tick(c, "gemm_ple_model_proj")) ||
         (rc = launch_ple_prep_rows(c->pf_proj, slice, c->ple_tab, c->ple_norm, c->pf_ids, M, Lc,
                                    1.0f / sqrtf((float)H), c->pf_ple, k.eps, st)) ||
@@ -1257,7 +1254,7 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
   for (int l = 0; l < Lc; ++l) {
     const Layer& ly = c->L[l];
     // attention block
-    if ((rc = gemm(q40_view(ly.qkv, c->qkv_rows, H), c->pf_xn, H, GEMM_F32, c->pf_qkv, nullptr, 0, nullptr, 0, ks_qkv)) ||
+    if ((rc = gemm(q40_view(ly.qkv, c->qkv_rows, H), c->pf_xn, H, GEMM_F32, c->pf_qkv, nullptr, 0, ks_qkv)) ||
         (rc = tick(c, "gemm_qkv")))
       return rc;
     if ((rc = launch_headprep_rows(c->pf_qkv, ks_qkv, (int64_t)M * c->qkv_rows, ly.q_norm, ly.k_norm, ly.global ? c->inv_global : c->inv_local,
@@ -1279,17 +1276,16 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
     pa.part = c->pf_apart;
     pa.part_bytes = c->pf_apart_bytes;
     if ((rc = launch_attn_prefill(pa, st)) || (rc = tick(c, "attn_prefill"))) return rc;
-    if ((rc = gemm(q40_view(ly.o, H, (int64_t)QH * HD), c->pf_attn, QH * HD, GEMM_F32, c->pf_y, nullptr, 0, nullptr,
-                   0, ks_o)) ||
+    if ((rc = gemm(q40_view(ly.o, H, (int64_t)QH * HD), c->pf_attn, QH * HD, GEMM_F32, c->pf_y, nullptr, 0, ks_o)) ||
         (rc = tick(c, "gemm_o")))
       return rc;
     // post-attention residual + FFN norm; gate/up + GeGLU; down
     if ((rc = launch_resnorm_rows(M, c->pf_h, c->pf_y, ks_o, MH, ly.post_attn, 1.0f, ly.ffn_norm, c->pf_xn, nullptr,
                                   H, k.eps, st)) ||
         (rc = tick(c, "resnorm_rows")) ||
-        (rc = gemm(q40_view(ly.gu, 2 * (int64_t)FF, H), c->pf_xn, H, GEMM_GLU, nullptr, c->pf_gg, FF, nullptr, 0, 1)) ||
+        (rc = gemm(q40_view(ly.gu, 2 * (int64_t)FF, H), c->pf_xn, H, GEMM_GLU, nullptr, c->pf_gg, FF, 1)) ||
         (rc = tick(c, "gemm_gate_up_geglu")) ||
-        (rc = gemm(q40_view(ly.down, H, FF), c->pf_gg, FF, GEMM_F32, c->pf_y, nullptr, 0, nullptr, 0, ks_d)) ||
+        (rc = gemm(q40_view(ly.down, H, FF), c->pf_gg, FF, GEMM_F32, c->pf_y, nullptr, 0, ks_d)) ||
         (rc = tick(c, "gemm_down")))
       return rc;
     // the last residual of the layer is followed by the next layer's input
@@ -1305,12 +1301,12 @@ int prefill_chunk(e4b_ctx* c, uint32_t p0, int M) {
       if ((rc = launch_resnorm_rows(M, c->pf_h, c->pf_y, ks_d, MH, ly.post_ffw, 1.0f, nullptr, c->pf_xn, nullptr, H,
                                     k.eps, st)) ||
           (rc = tick(c, "resnorm_rows")) ||
-          (rc = gemm(q40_view(ly.pg, PD, H), c->pf_xn, H, GEMM_F32, c->pf_y, nullptr, 0, nullptr, 0, ks_pg)) ||
+          (rc = gemm(q40_view(ly.pg, PD, H), c->pf_xn, H, GEMM_F32, c->pf_y, nullptr, 0, ks_pg)) ||
           (rc = tick(c, "gemm_ple_gate")) ||
           (rc = launch_gelu_mul_rows(c->pf_y, ks_pg, (int64_t)M * PD, M, PD, c->pf_ple + (int64_t)l * PD, NP, c->pf_gp,
                                      st)) ||
           (rc = tick(c, "gelu_mul_rows")) ||
-          (rc = gemm(q40_view(ly.pp_rm, H, PD), c->pf_gp, PD, GEMM_F32, c->pf_y, nullptr, 0, nullptr, 0, 1)) ||
+          (rc = gemm(q40_view(ly.pp_rm, H, PD), c->pf_gp, PD, GEMM_F32, c->pf_y, nullptr, 0, 1)) ||
           (rc = tick(c, "gemm_ple_proj")) ||
           (rc = launch_resnorm_rows(M, c->pf_h, c->pf_y, 1, 0, ly.post_norm, ly.scale, w_next, x_next, xlo_next, H,
                                     k.eps, st)) ||

@@ -6,8 +6,8 @@
 //
 //   Y[m][n] = sum_k X[m][k] W[n][k],  W q4_0 [N][K] (repacked planes),
 //   X f16 [M][K] row-major (row stride ldx), Y f32 [M][N]; epilogues: split-K
-//   partial slices (Y + z M N, summed by the consumer), the GeGLU over
-//   W = [gate; up] to f16 [M][FF] = gelu(gate) * up, or f16 gelu(y) * mul.
+//   partial slices (Y + z M N, summed by the consumer), or the GeGLU over
+//   W = [gate; up] to f16 [M][FF] = gelu(gate) * up.
 //
 // v_mfma_f32_32x32x16_f16 with A = a 32-token x 16-k slice of X and B = the
 // 16-k x 32-row slice of W^T: lane l holds A[l % 32][8 (l / 32) + t] (t < 8),
@@ -361,10 +361,7 @@ DEV void gemm_tile(const GemmArgs& a, int nb, int nbs, int bx, int by, u32x4* bu
       for (int u = 0; u < NT; ++u) {
         const int64_t n = c0 + (u * RW + rw) * 32 + l32;
         if (n >= units) continue;
-        if constexpr (EPI == GEMM_GELU_MUL)
-          a.Yh[m * units + n] = f2h(gelu_sigmoid(v[u]) * a.mul[m * a.mul_ld + n]);
-        else
-          a.Y[((int64_t)kz * a.M + m) * units + n] = v[u];
+        a.Y[((int64_t)kz * a.M + m) * units + n] = v[u];
       }
     }
   };

@@ -31,11 +31,8 @@ using gemm::VariantSet;
 VariantSet variants(int epi, bool grp, bool aligned) {
   using namespace gemm;
   if (grp) return variants_grp(epi == GEMM_GLU, aligned);
-  switch (epi) {
-    case GEMM_GLU: return aligned ? variants_glu() : variants_glu_odd();
-    case GEMM_GELU_MUL: return aligned ? variants_mul() : variants_mul_odd();
-    default: return aligned ? variants_f32() : variants_f32_odd();
-  }
+  if (epi == GEMM_GLU) return aligned ? variants_glu() : variants_glu_odd();
+  return aligned ? variants_f32() : variants_f32_odd();
 }
 
 // Estimated microseconds of a launch: which tile is best depends on how the
@@ -139,9 +136,6 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
         return e4b_fail(E4B_EINVAL, "q4_0 GEMM: GeGLU needs 2*ff rows");
       units = a.ff;
       break;
-    case GEMM_GELU_MUL:
-      if (!a.Yh || !a.mul || grp) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: GELU-multiply needs yh and mul");
-      break;
     default: return e4b_fail(E4B_EINVAL, "q4_0 GEMM: epilogue %d", a.epi);
   }
   // blocks per split-K slice; the consumer sums exactly `ks` slices, so every
@@ -171,7 +165,6 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
       c.X = a.X + m0 * a.ldx;
       if (a.Y) c.Y = a.Y + m0 * units;
       if (a.Yh) c.Yh = a.Yh + m0 * units;
-      if (a.mul) c.mul = a.mul + m0 * a.mul_ld;
       const Variant& v = choose(set, c.epi, units, W.nb, c.M, 1, nullptr);
       v.go(c, nbs, (unsigned)((c.M + 32 * v.T - 1) / (32 * v.T)), 1, st);
     }

@@ -1,4 +1,4 @@
-// k_gemm_glu.hip -- the q4_0 GEMM's GeGLU and GELU-multiply variants.
+// k_gemm_glu.hip -- the q4_0 GEMM's GeGLU variants.
 #include "gemm_variants.h"
 
 namespace gemm {
@@ -10,15 +10,6 @@ VariantSet variants_glu() {
       GEMM_VARIANT(4, 2, 8, 1, 2, GEMM_GLU, false, true, 230), GEMM_VARIANT(2, 2, 4, 2, 2, GEMM_GLU, false, true, 170),
       GEMM_VARIANT(2, 2, 2, 4, 2, GEMM_GLU, false, true, 170), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, false, true, 170),
       GEMM_VARIANT(1, 2, 1, 4, 2, GEMM_GLU, false, true, 110), GEMM_VARIANT(1, 2, 1, 8, 2, GEMM_GLU, false, true, 110),
-  };
-  return {v, (int)(sizeof(v) / sizeof(v[0]))};
-}
-
-VariantSet variants_mul() {
-  static const Variant v[] = {
-      GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_GELU_MUL, false, true, 108),
-      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_GELU_MUL, false, true, 76),
-      GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_GELU_MUL, false, true, 76),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }

@@ -21,11 +21,4 @@ VariantSet variants_glu_odd() {
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }
 
-VariantSet variants_mul_odd() {
-  static const Variant v[] = {
-      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_GELU_MUL, false, false, 76),
-  };
-  return {v, (int)(sizeof(v) / sizeof(v[0]))};
-}
-
 }  // namespace gemm

@@ -10,8 +10,7 @@
 //   grouped GEMMs       expert gate/up + GeGLU and expert down on the matrix
 //                       cores (k_gemm.hip grouped mode): each tile reads its
 //                       expert's rows once for up to 64 draws
-//   dense branch        gate|up GEMM in K slices, k_geglu_rows, down GEMM in
-//                       K slices over all M tokens
+//   dense branch        gate|up + GeGLU GEMM, down GEMM (K slices) over all M tokens
 //   k_moe_combine_rows  moe[m] = sum_k w_k down_sorted[pos(m, k)], in k order,
 //                       and the dense down's K slices summed
 //   tail                the decode tail over token rows
@@ -63,22 +62,6 @@ __global__ __launch_bounds__(1024) void k_moe_group(const uint32_t* __restrict__
       tiles[toff[e] + j] = make_int4(e, off[e] + j * kTileRows, min(kTileRows, cnt[e] - j * kTileRows), 0);
 }
 
-// out[m][j] = f16(gelu(gate) * up) of the dense branch, gate and up each the
-// sum of the ks split-K slices of the gate|up GEMM (rows j and FF + j), in
-// slice order; the arithmetic of the GEMM's GeGLU epilogue after that sum
-__global__ __launch_bounds__(256) void k_geglu_rows(const float* __restrict__ part, int ks, int64_t slice, int FF,
-                                                    uint16_t* __restrict__ out) {
-  const int m = blockIdx.y, j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= FF) return;
-  const float* p = part + (int64_t)m * 2 * FF + j;
-  float g = p[0], u = p[FF];
-  for (int s = 1; s < ks; ++s) {
-    g += p[s * slice];
-    u += p[s * slice + FF];
-  }
-  out[(int64_t)m * FF + j] = f2h(gelu_tanh(g) * u);
-}
-
 // moe[m][i] = sum_k w[m][k] * down[pos[m K + k]][i], in slot order
 // (and dense[m] = the sum of the dense down GEMM's dks K slices of row m, in
 // slice order)
@@ -124,7 +107,7 @@ size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* 
   uint8_t* p_g = take(P * FF * 2);
   uint8_t* p_d = take(P * H * 4);
   uint8_t* p_gd = take((size_t)M * FF2 * 2);
-  uint8_t* p_gdp = take((size_t)kMoePfDenseKs * M * (2 * FF2 > H ? 2 * FF2 : H) * 4);
+  uint8_t* p_ddp = take((size_t)kMoePfDenseKs * M * H * 4);
   uint8_t* p_dense = take((size_t)M * H * 4);
   uint8_t* p_moe = take((size_t)M * H * 4);
   if (b) {
@@ -141,7 +124,7 @@ size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* 
     b->g_sorted = (uint16_t*)p_g;
     b->d_sorted = (float*)p_d;
     b->g_dense = (uint16_t*)p_gd;
-    b->gd_part = (float*)p_gdp;
+    b->dd_part = (float*)p_ddp;
     b->dense_out = (float*)p_dense;
     b->moe_out = (float*)p_moe;
   }
@@ -194,28 +177,29 @@ int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipS
   g.gather = nullptr;
   g.gather_div = 1;
   if ((rc = launch_q40_gemm(g, st))) return rc;
-  // dense branch over all tokens: gate|up in K slices, then the GeGLU rows
+  // dense branch over all tokens; the down projection's K slices are summed
+  // by the combine
   GemmArgs d{};
   d.W = a.dense_gu;
   d.X = b.xd;
   d.M = M;
   d.ldx = H;
-  d.epi = GEMM_F32;
-  d.Y = b.gd_part;
-  d.ks = q40_gemm_kslices(a.dense_gu.nb, kMoePfDenseKs);
+  d.epi = GEMM_GLU;
+  d.Yh = b.g_dense;
+  d.ff = FF2;
+  d.ks = 1;
   if ((rc = launch_q40_gemm(d, st))) return rc;
-  hipLaunchKernelGGL(k_geglu_rows, dim3((FF2 + 255) / 256, M), dim3(256), 0, st, b.gd_part, d.ks,
-                     (int64_t)M * 2 * FF2, FF2, b.g_dense);
-  E4B_HIP(hipGetLastError());
   d.W = a.dense_down;
   d.X = b.g_dense;
   d.ldx = FF2;
   d.epi = GEMM_F32;
-  d.Y = b.gd_part;  // the down's K slices reuse the gate|up partials' space
-  d.ks = q40_gemm_kslices(a.dense_down.nb, kMoePfDenseKs);
+  d.Y = b.dd_part;
+  d.Yh = nullptr;
+  d.ff = 0;
+  d.ks = q40_gemm_best_kslices(H, a.dense_down.nb, M, kMoePfDenseKs);
   if ((rc = launch_q40_gemm(d, st))) return rc;
   hipLaunchKernelGGL(k_moe_combine_rows, dim3((H + 255) / 256, M), dim3(256), 0, st, b.d_sorted, b.pos, b.topk_w, H,
-                     b.moe_out, b.gd_part, d.ks, (int64_t)M * H, b.dense_out);
+                     b.moe_out, b.dd_part, d.ks, (int64_t)M * H, b.dense_out);
   E4B_HIP(hipGetLastError());
   return launch_moe_tail_rows(a, M, st);
 }

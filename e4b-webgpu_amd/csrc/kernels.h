@@ -119,7 +119,6 @@ int launch_q40_gemm(const Q40Mat& W, const uint16_t* X, int M, float* Y, uint16_
 enum GemmEpi {
   GEMM_F32 = 0,       // Y[(z M + m) rows + n]: split-K slice z of ks (ks = 1: the product)
   GEMM_GLU = 1,       // rows [0,ff) gate, [ff,2ff) up: Yh[m ff + i] = f16(gelu(g) * u)
-  GEMM_GELU_MUL = 2,  // Yh[m rows + n] = f16(gelu(y) * mul[m mul_ld + n])
 };
 struct GemmArgs {
   Q40Mat W;
@@ -129,8 +128,6 @@ struct GemmArgs {
   float* Y;
   uint16_t* Yh;
   int64_t ff;
-  const float* mul;
-  int64_t mul_ld;
   int ks;             // split-K slices (GEMM_F32)
   // grouped mode (the expert-indexed MoE prefill; tiles != null): blockIdx.y
   // picks tiles[y] = (group g, first row r0, rows n <= 64) of the M sorted
