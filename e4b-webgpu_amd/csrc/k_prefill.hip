@@ -287,16 +287,32 @@ __global__ __launch_bounds__(64) void k_headprep_rows(const float* __restrict__ 
 //   After the online-softmax update each lane holds P^T for its query
 //   (column l % 16) and 8 keys: 4 (l / 16) + r of sub-tile 0 and 16 + 4 (l /
 //   16) + r of sub-tile 1 -- exactly a B operand of a 32-key MFMA when the A
-//   operand (V^T, 16 dims x 32 keys, read from a transposed V tile in LDS)
-//   uses the same key order.  O^T (dims x queries) accumulates P_hi and
-//   P_lo (P = P_hi + P_lo) against V in f32, so every product is as exact
-//   as the decode kernel's f32 arithmetic.
+//   operand (V^T, 16 dims x 32 keys) uses the same key order.  O^T (dims x
+//   queries) accumulates P_hi and P_lo (P = P_hi + P_lo) against V in f32, so
+//   every product is as exact as the decode kernel's f32 arithmetic.
+//
+// What bounds it: latency.  A workgroup's matrix work is a microsecond or
+// two; the rest was each tile's load, waited for in full, and the V
+// transposition in registers, whose LDS stores hit one bank 16 ways.  So K
+// and V rows go row-major from memory straight into LDS, one tile ahead in a
+// second buffer, xor-swizzled by row (a row is 512 bytes: without it the 16
+// rows of a fragment share their banks), and V^T is read with the transposing
+// ds_read_b64_tr_b16: a group of 16 lanes reads 4 keys x 16 dims, lane i
+// addressing key i / 4, dims 4 (i % 4), and receives dim i of the 4 keys.
+// Per call with its merge of the splits, before -> now: 512 queries x 8 heads
+// over a window of 512 keys 31.2 -> 25.7 us, at the end of 4096 keys 86.9 ->
+// 60 us, 512 x 16 heads over 8 KV heads 43.3 -> 33.9 us, one query over 3001
+// keys 37.6 -> 25.7 us.  Tried and left out, all at the same time or slower:
+// more of a tile's fragments read ahead into registers, four tiles in flight
+// with one workgroup per CU (29.9 us), the loop unrolled over both buffers.
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
+typedef __fp16 tr4 __attribute__((__vector_size__(8)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) tr4 lds_tr4;
 
-constexpr int kKT = 32;            // keys per tile
-// halfs per K row in LDS: the head dim + 8
-constexpr int kVtStride = kKT + 8; // halfs per transposed V row in LDS
+constexpr int kKT = 32;              // keys per tile
 constexpr int kPfAttnMaxSplits = 8;  // key splits per query tile
 constexpr int kPfAttnMinSplit = 128; // keys per split at least (a multiple of kKT)
 
@@ -308,21 +324,31 @@ DEV void split8(const float (&v)[8], h8v& hi, h8v& lo) {
     lo[t] = (_Float16)(v[t] - (float)a);
   }
 }
+// max / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48
+DEV float quad_max(float v) {
+  float t = v;
+  swapx32(v, t);
+  v = fmaxf(v, t);
+  t = v;
+  swapx16(v, t);
+  return fmaxf(v, t);
+}
+DEV float quad_sum(float v) { return xsum_step<16>(xsum_step<32>(v)); }
 
 // Head dim 512 (GQA 8, the A4B full layers): blockIdx.x also picks one of
 // the two sets of 4 heads and one of the two 256-dim halves of V, so a
 // workgroup holds 4 heads' O for 256 dims; both V halves compute the scores.
 template <int GQA, int HD = 256>
-__global__ __launch_bounds__(256) void k_attn_prefill(PrefillAttnArgs A) {
+__global__ __launch_bounds__(256, HD == 256 ? 2 : 1) void k_attn_prefill(PrefillAttnArgs A) {
   static_assert((HD == 256 && GQA <= 4) || (HD == 512 && GQA == 8), "head dim 256 (GQA <= 4) or 512 (GQA 8)");
   constexpr int QS = GQA >= 4 ? 1 : 4 / GQA;  // 16-query sub-tiles per workgroup
   constexpr int NVH = HD / 256;               // 256-dim V halves
   constexpr int NHS = GQA > 4 ? GQA / 4 : 1;  // sets of 4 heads
   constexpr int WG = GQA > 4 ? GQA : 4;       // partial units per (group, tile, split)
-  constexpr int KST = HD + 8;                 // halfs per K row in LDS
-  __shared__ __align__(16) uint16_t ks[kKT * KST];
-  __shared__ __align__(16) uint16_t vt[256 * kVtStride];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int KP = HD / 8;                  // 16-byte pieces of a K row
+  constexpr int KB = kKT * KP, VB = kKT * 32; // and of a K and a V tile
+  __shared__ __align__(16) uint4 bufs[2][KB + VB];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = blockIdx.x / (NHS * NVH), hs = (blockIdx.x / NVH) % NHS, vh = blockIdx.x % NVH;
   const int t0 = blockIdx.y * 16 * QS, q0 = t0 + 16 * (GQA >= 4 ? 0 : wave / GQA);
   const int hg = GQA >= 4 ? 4 * hs + wave : wave % GQA;  // head within the group
@@ -336,77 +362,84 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillAttnArgs A) {
   const int P0 = (int)A.p0 + t0, P1 = (int)A.p0 + min(t0 + 16 * QS, M) - 1;
   const int W = A.window;
   const int klo = W > 0 ? max(0, P0 - W + 1) : 0;
-  const uint16_t* kc = A.kc + (int64_t)g * A.slots * HD;
-  const uint16_t* vc = A.vc + (int64_t)g * A.slots * HD + 256 * vh;
   const int NS = gridDim.z, sp = blockIdx.z;
   const int kstart = NS > 1 ? klo + sp * A.kspl : klo;
   if (kstart > P1) return;  // this tile needs fewer splits (uniform per workgroup)
   const int kend = NS > 1 ? min(P1, kstart + A.kspl - 1) : P1;
-
-  // Q^T as the B operand: step s covers dims 32 s + 8 qq .. + 8
+  const uint16_t* kg = A.kc + (int64_t)g * A.slots * HD;
+  const uint16_t* vg = A.vc + (int64_t)g * A.slots * HD + 256 * vh;
+  auto copy16 = [](const uint16_t* base, uint4* dst, int off) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00020000),
+                                             (lds_void*)dst, 16, off, 0, 0, 0);
+  };
+  // A tile is keys kb .. kb + last: 32, or as many as are left of the split or
+  // up to the end of the ring, so that its rows lie one behind the other from
+  // slot sb (rows past the last repeat it and are masked)
+  auto tile_last = [&](int kb, int sb) { return min(kKT - 1, min(kend - kb, A.slots - 1 - sb)); };
+  // a wave copies 1 KB at a time, 64 / KP K rows or 2 V rows
+  auto issue = [&](uint4* buf, int sb, int last) __attribute__((always_inline)) {
+    const uint16_t *kt = kg + (int64_t)sb * HD, *vt = vg + (int64_t)sb * HD;
+#pragma unroll
+    for (int i = 0; i < KB / 256; ++i) {
+      const int p = (4 * i + wave) * 64 + lane, r = p / KP;
+      copy16(kt, buf + (4 * i + wave) * 64, min(r, last) * (HD * 2) + ((p % KP) ^ (r & 15)) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < VB / 256; ++i) {
+      const int p = (4 * i + wave) * 64 + lane, r = p / 32;
+      copy16(vt, buf + KB + (4 * i + wave) * 64, min(r, last) * (HD * 2) + ((p % 32) ^ ((r & 15) << 1)) * 16);
+    }
+  };
+  int kb = kstart, sb = W > 0 ? kstart % A.slots : kstart, last = tile_last(kb, sb);
+  // Q^T as the B operand: step s covers dims 32 s + 8 qq .. + 8.  All of the
+  // row's loads go out first, then the first tile's copies, then the splits.
   constexpr int QST = HD / 32;  // score steps
   h8v qh_[QST], ql_[QST];
   {
-    const float* qrow = A.q + ((int64_t)min(qi, M - 1) * A.qh + head) * HD;
+    const float4* qrow = reinterpret_cast<const float4*>(A.q + ((int64_t)min(qi, M - 1) * A.qh + head) * HD) + 2 * qq;
+    constexpr int QB = 8;  // steps per batch
 #pragma unroll
-    for (int s = 0; s < QST; ++s) {
-      const float4 a = *reinterpret_cast<const float4*>(qrow + 32 * s + 8 * qq);
-      const float4 b = *reinterpret_cast<const float4*>(qrow + 32 * s + 8 * qq + 4);
-      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      split8(v, qh_[s], ql_[s]);
+    for (int b = 0; b < QST; b += QB) {
+      f4v raw[QB][2];
+#pragma unroll
+      for (int s = 0; s < QB; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) raw[s][i] = __builtin_bit_cast(f4v, qrow[8 * (b + s) + i]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b == 0) {
+        issue(bufs[0], sb, last);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int s = 0; s < QB; ++s) {
+        const float v[8] = {raw[s][0][0], raw[s][0][1], raw[s][0][2], raw[s][0][3],
+                            raw[s][1][0], raw[s][1][1], raw[s][1][2], raw[s][1][3]};
+        split8(v, qh_[b + s], ql_[b + s]);
+      }
     }
   }
   f4v o[16];
 #pragma unroll
   for (int dt = 0; dt < 16; ++dt) o[dt] = f4v{0.f, 0.f, 0.f, 0.f};
   float mrun = -3.0e38f, lrun = 0.f;
+  // LDS addresses: K row 16 kt + j, piece 4 s + qq; V key 4 qq + j / 4 (+ 16),
+  // dims 16 dt + 4 (j % 4)
+  const int kr0 = j * KP, vrow = 4 * qq + (j >> 2);
+  const int va0 = KB * 16 + vrow * 512 + ((j & 3) >> 1) * 16 + (j & 1) * 8;
 
-  for (int kb = kstart; kb <= kend; kb += kKT) {
-    // stage keys kb .. kb + 31 (rows past P1 repeat row P1; they are masked)
-    lds_sync();
-    {
-      const int t = threadIdx.x;
-      // K: 8 threads per row, HD / 8 halfs each
-      const int kr = t >> 3, part = t & 7;
-      const int kp = min(kb + kr, P1);
-      const int64_t sk = W > 0 ? (int64_t)(kp % A.slots) : (int64_t)kp;
-      const uint4* srck = reinterpret_cast<const uint4*>(kc + sk * HD + (HD / 8) * part);
-      uint4* dstk = reinterpret_cast<uint4*>(ks + kr * KST + (HD / 8) * part);
+  auto tile = [&](const uint4* buf, int kb, int last) __attribute__((always_inline)) {
+    // S^T for the two 16-key sub-tiles, hi and lo products apart: four chains
+    f4v sc[2][2];
 #pragma unroll
-      for (int i = 0; i < HD / 64; ++i) dstk[i] = srck[i];
-      // V: thread (key pair kp2, dim chunk dc) transposes 2 keys x 16 dims
-      const int kp2 = t >> 4, dc = t & 15;
-      const int pa = min(kb + 2 * kp2, P1), pb = min(kb + 2 * kp2 + 1, P1);
-      const int64_t sa = W > 0 ? (int64_t)(pa % A.slots) : (int64_t)pa;
-      const int64_t sb = W > 0 ? (int64_t)(pb % A.slots) : (int64_t)pb;
-      const uint4* va = reinterpret_cast<const uint4*>(vc + sa * HD + 16 * dc);
-      const uint4* vb = reinterpret_cast<const uint4*>(vc + sb * HD + 16 * dc);
-      const uint4 a0 = va[0], a1 = va[1], b0 = vb[0], b1 = vb[1];
-      const uint32_t aw[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-      const uint32_t bw[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+    for (int kt = 0; kt < 2; ++kt) sc[kt][0] = sc[kt][1] = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t lo2 = (aw[i] & 0xffffu) | (bw[i] << 16);
-        const uint32_t hi2 = (aw[i] >> 16) | (bw[i] & 0xffff0000u);
-        *reinterpret_cast<uint32_t*>(vt + (16 * dc + 2 * i) * kVtStride + 2 * kp2) = lo2;
-        *reinterpret_cast<uint32_t*>(vt + (16 * dc + 2 * i + 1) * kVtStride + 2 * kp2) = hi2;
+    for (int s = 0; s < QST; ++s)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const h8v ka = __builtin_bit_cast(h8v, buf[kr0 + 16 * kt * KP + ((4 * s + qq) ^ j)]);
+        sc[kt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh_[s], sc[kt][0], 0, 0, 0);
+        sc[kt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql_[s], sc[kt][1], 0, 0, 0);
       }
-    }
-    lds_sync();
-    // S^T for the two 16-key sub-tiles
-    f4v sc[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      f4v d = {0.f, 0.f, 0.f, 0.f};
-      const uint16_t* krow = ks + (16 * kt + j) * KST + 8 * qq;
-#pragma unroll
-      for (int s = 0; s < QST; ++s) {
-        const h8v ka = __builtin_bit_cast(h8v, *reinterpret_cast<const uint4*>(krow + 32 * s));
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh_[s], d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql_[s], d, 0, 0, 0);
-      }
-      sc[kt] = d;
-    }
     // mask, online softmax (per query column; its 32 scores sit in the four
     // lanes j, j + 16, j + 32, j + 48)
     float p[8];
@@ -416,12 +449,11 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillAttnArgs A) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int kp = kb + 16 * kt + 4 * qq + r;
-        const bool live = qi < M && kp <= qp && kp <= P1 && (W == 0 || kp > qp - W);
-        p[4 * kt + r] = live ? sc[kt][r] : -3.0e38f;
+        const bool live = qi < M && kp <= qp && kp <= kb + last && (W == 0 || kp > qp - W);
+        p[4 * kt + r] = live ? sc[kt][0][r] + sc[kt][1][r] : -3.0e38f;
         mx = fmaxf(mx, p[4 * kt + r]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = quad_max(mx);
     const float mnew = fmaxf(mrun, mx);
     const float alpha = __expf(mrun - mnew);
     float ps = 0.f;
@@ -430,24 +462,54 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillAttnArgs A) {
       p[i] = p[i] > -1.0e38f ? __expf(p[i] - mnew) : 0.f;
       ps += p[i];
     }
-    ps += __shfl_xor(ps, 16, 64);
-    ps += __shfl_xor(ps, 32, 64);
+    ps = quad_sum(ps);
     lrun = lrun * alpha + ps;
     mrun = mnew;
+    // (alpha is 1 in every lane unless a query met a new maximum)
+    if (__any(alpha != 1.f)) {
 #pragma unroll
-    for (int dt = 0; dt < 16; ++dt) o[dt] *= alpha;
+      for (int dt = 0; dt < 16; ++dt) o[dt] *= alpha;
+    }
     h8v phi, plo;
     split8(p, phi, plo);
     // O^T += V^T P^T: A = V^T rows 16 dt + j, keys 4 qq .. +3 and 16 + 4 qq .. +3
+    auto ldv = [&](int dt, int half) {
+      const int a = va0 + half * (16 * 512) + ((2 * dt) ^ (vrow << 1)) * 16;
+      return __builtin_bit_cast(u2v, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+                                         (lds_tr4*)(reinterpret_cast<const char*>(buf) + a)));
+    };
 #pragma unroll
-    for (int dt = 0; dt < 16; ++dt) {
-      const uint16_t* vrow = vt + (16 * dt + j) * kVtStride;
-      const uint2 va = *reinterpret_cast<const uint2*>(vrow + 4 * qq);
-      const uint2 vb = *reinterpret_cast<const uint2*>(vrow + 16 + 4 * qq);
-      const h8v vv = __builtin_bit_cast(h8v, make_uint4(va.x, va.y, vb.x, vb.y));
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, phi, o[dt], 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, plo, o[dt], 0, 0, 0);
+    for (int d2 = 0; d2 < 16; d2 += 2) {
+      h8v vv[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const u2v va = ldv(d2 + e, 0), vb = ldv(d2 + e, 1);
+        vv[e] = __builtin_bit_cast(h8v, make_uint4(va.x, va.y, vb.x, vb.y));
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) o[d2 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[e], phi, o[d2 + e], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) o[d2 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv[e], plo, o[d2 + e], 0, 0, 0);
     }
+  };
+  // (no alias between the two buffers: the copies into one need no wait
+  // before the reads of the other)
+  auto step = [&](const uint4* __restrict__ cur, uint4* __restrict__ nxt, int nkb, int nsb,
+                  int nlast) __attribute__((always_inline)) {
+    if (nkb <= kend) issue(nxt, nsb, nlast);
+    tile(cur, kb, last);
+  };
+  for (int b = 0;; b ^= 1) {
+    // every wave's copies of the tile have landed, and every wave is done
+    // with the buffer the next copies overwrite
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    lds_sync();
+    const int nkb = kb + last + 1, nsb = sb + last + 1 < A.slots ? sb + last + 1 : 0, nlast = tile_last(nkb, nsb);
+    step(bufs[b], bufs[b ^ 1], nkb, nsb, nlast);
+    if (nkb > kend) break;
+    kb = nkb;
+    sb = nsb;
+    last = nlast;
   }
   if (qi >= M) return;
   if (NS > 1) {
@@ -652,3 +714,4 @@ int launch_attn_prefill(PrefillAttnArgs a, hipStream_t st) {
   E4B_HIP(hipGetLastError());
   return E4B_OK;
 }
+
