@@ -822,12 +822,7 @@ __global__ __launch_bounds__(256) void k_moe_tail(MoeArgs A) {
   E4B_TRACE_SCOPE(trace_tag(TR_MOE_TAIL, 0));
   __shared__ float red[4];
   const int H = A.H;
-  // token row blockIdx.x of a batch (one block in the decode step)
-  const int64_t ro = (int64_t)blockIdx.x * H;
-  A.h = (A.attn_o ? A.h1 : A.h) + ro;
-  A.dense_out += ro;
-  A.moe_out += ro;
-  A.h_out += ro;
+  A.h = A.attn_o ? A.h1 : A.h;
   // every input requested before the first reduction waits
   float d[kTailPer], m[kTailPer], w1[kTailPer], w2[kTailPer], hv[kTailPer], wp[kTailPer];
 #pragma unroll
@@ -920,13 +915,6 @@ int launch_moe_router_rows(const MoeArgs& A, int M, hipStream_t st) {
 int launch_moe_topk_rows(const MoeArgs& A, int M, hipStream_t st) {
   if (A.E < K || A.E > 256 || M < 1) return e4b_fail(E4B_EINVAL, "top-8 rows: E=%d M=%d", A.E, M);
   hipLaunchKernelGGL(k_moe_topk, dim3(M), dim3(64), 0, st, A);
-  E4B_HIP(hipGetLastError());
-  return E4B_OK;
-}
-
-int launch_moe_tail_rows(const MoeArgs& A, int M, hipStream_t st) {
-  if (A.H > 256 * kTailPer || M < 1) return e4b_fail(E4B_EINVAL, "MoE tail rows: H=%d M=%d", A.H, M);
-  hipLaunchKernelGGL(k_moe_tail, dim3(M), dim3(256), 0, st, A);
   E4B_HIP(hipGetLastError());
   return E4B_OK;
 }

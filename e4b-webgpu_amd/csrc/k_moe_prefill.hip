@@ -11,9 +11,8 @@
 //                       cores (k_gemm.hip grouped mode): each tile reads its
 //                       expert's rows once for up to 64 draws
 //   dense branch        gate|up + GeGLU GEMM, down GEMM (K slices) over all M tokens
-//   k_moe_combine_rows  moe[m] = sum_k w_k down_sorted[pos(m, k)], in k order,
-//                       and the dense down's K slices summed
-//   tail                the decode tail over token rows
+//   k_moe_combine_tail  moe[m] = sum_k w_k down_sorted[pos(m, k)], in k order,
+//                       the dense down's K slices summed, and the decode tail
 #include "../../include/e4b.h"
 #include "kernels.h"
 #include "moe.h"
@@ -22,65 +21,138 @@
 namespace {
 
 constexpr int K = kMoeTopK;
+constexpr int kMoePfMaxTokens = 1024;
 constexpr int kTileRows = 64;  // the grouped GEMM's row tile
 
 // one workgroup: histogram of the draws' experts in LDS, exclusive scan,
 // placement (list[slot] = draw, pos[draw] = slot) and the tile table.  The
 // order of draws inside an expert's run depends on LDS atomics; every output
 // row is computed from its own input row only, so results do not.
+//
+// All latency.  A thread keeps its draws (at most 8) and the rank that the
+// histogram's atomic returned for each, so the picks are read once and one
+// round of atomics places them; rows and tiles are scanned together (16 bits
+// each) by lane shifts.
+// (One thread scanning 128 experts, the picks read twice: 8.8 us over 512
+// tokens; now 5.4.)
 __global__ __launch_bounds__(1024) void k_moe_group(const uint32_t* __restrict__ topk_idx, int npairs, int E,
                                                     uint32_t* __restrict__ list, uint32_t* __restrict__ pos,
                                                     int4* __restrict__ tiles, int* __restrict__ ntiles) {
-  __shared__ int cnt[256], off[256], fill[256], toff[256];
-  const int t = threadIdx.x;
+  constexpr int D = kMoePfMaxTokens * K / 1024;  // draws per thread
+  __shared__ int cnt[256];
+  __shared__ uint32_t off[256];  // rows before the expert, tiles before it << 16
+  __shared__ uint32_t wtot[4];
+  const int t = threadIdx.x, lane = t & 63;
+  int e[D], rank[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) e[i] = t + 1024 * i < npairs ? min((int)topk_idx[t + 1024 * i], E - 1) : -1;
+  if (t < 256) cnt[t] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < D; ++i) rank[i] = e[i] >= 0 ? atomicAdd(&cnt[e[i]], 1) : 0;
+  __syncthreads();
+  uint32_t own = 0, sum = 0;
   if (t < 256) {
-    cnt[t] = 0;
-    fill[t] = 0;
-  }
-  __syncthreads();
-  for (int p = t; p < npairs; p += 1024) atomicAdd(&cnt[min((int)topk_idx[p], E - 1)], 1);
-  __syncthreads();
-  if (t == 0) {
-    int o = 0, tt = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o;
-      toff[e] = tt;
-      o += cnt[e];
-      tt += (cnt[e] + kTileRows - 1) / kTileRows;
+    const int n = cnt[t];
+    own = (uint32_t)n | (uint32_t)((n + kTileRows - 1) / kTileRows) << 16;
+    sum = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t o = __shfl_up(sum, d, 64);
+      sum += lane >= d ? o : 0u;
     }
-    *ntiles = tt;
+    if (lane == 63) wtot[t >> 6] = sum;
   }
   __syncthreads();
-  for (int p = t; p < npairs; p += 1024) {
-    const int e = min((int)topk_idx[p], E - 1);
-    const int s = off[e] + atomicAdd(&fill[e], 1);
-    list[s] = (uint32_t)p;
-    pos[p] = (uint32_t)s;
+  if (t < 256) {
+    for (int w = 0; w < t >> 6; ++w) sum += wtot[w];
+    const uint32_t ex = sum - own;
+    off[t] = ex;
+    const int n = (int)(own & 0xffffu), row = (int)(ex & 0xffffu), tile = (int)(ex >> 16);
+    for (int j = 0; j * kTileRows < n; ++j)
+      tiles[tile + j] = make_int4(t, row + j * kTileRows, min(kTileRows, n - j * kTileRows), 0);
+    if (t == 255) *ntiles = (int)(sum >> 16);
   }
-  for (int e = t; e < E; e += 1024)
-    for (int j = 0; j * kTileRows < cnt[e]; ++j)
-      tiles[toff[e] + j] = make_int4(e, off[e] + j * kTileRows, min(kTileRows, cnt[e] - j * kTileRows), 0);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    if (e[i] >= 0) {
+      const int p = t + 1024 * i, s = (int)(off[e[i]] & 0xffffu) + rank[i];
+      list[s] = (uint32_t)p;
+      pos[p] = (uint32_t)s;
+    }
 }
 
-// moe[m][i] = sum_k w[m][k] * down[pos[m K + k]][i], in slot order
-// (and dense[m] = the sum of the dense down GEMM's dks K slices of row m, in
-// slice order)
-__global__ __launch_bounds__(256) void k_moe_combine_rows(const float* __restrict__ down,
-                                                          const uint32_t* __restrict__ pos,
-                                                          const float* __restrict__ topk_w, int H,
-                                                          float* __restrict__ moe, const float* __restrict__ dpart,
-                                                          int dks, int64_t dslice, float* __restrict__ dense) {
-  const int m = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= H) return;
-  const int64_t o = (int64_t)m * H + i;
-  float ds = dpart[o];
-  for (int s = 1; s < dks; ++s) ds += dpart[s * dslice + o];
-  float acc = 0.f;
+// One workgroup per token row m: moe[m] = sum_k w[m][k] down[pos[m K + k]], in
+// slot order, dense[m] = the sum of the dense down GEMM's dks K slices, in
+// slice order, and the decode tail (k_moe_tail) of the two, which stay in
+// registers.  Bounded by the reads of the K sorted rows: a thread owns four
+// adjacent elements, so that all its loads are in flight at once (12 single
+// elements a thread, in a loop, took 22 us over 512 rows).
+// Measured over 512 rows of 2816: 13.4 us, in two kernels 9.9 + 6.6 and the
+// launch between them (the layer, with the grouping above, 260 -> 247).
+constexpr int kCtThreads = 768;  // 4 elements each: H <= 3072
+DEV float4 ld4(const float* p) {  // 4-byte aligned
+  float4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+DEV float4 fma4(float s, float4 a, float4 b) {
+  return make_float4(fmaf(s, a.x, b.x), fmaf(s, a.y, b.y), fmaf(s, a.z, b.z), fmaf(s, a.w, b.w));
+}
+DEV float dot4(float4 a) { return fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, a.w * a.w))); }
+DEV float ct_sum(float v, float* red) {  // over the workgroup; red: one float a wave
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  lds_sync();
+  float s = 0.f;
 #pragma unroll
-  for (int k = 0; k < K; ++k) acc = fmaf(topk_w[m * K + k], down[(int64_t)pos[m * K + k] * H + i], acc);
-  moe[o] = acc;
-  dense[o] = ds;
+  for (int w = 0; w < kCtThreads / 64; ++w) s += red[w];
+  return s;
+}
+__global__ __launch_bounds__(kCtThreads) void k_moe_combine_tail(MoeArgs A, const float* __restrict__ down,
+                                                                 const uint32_t* __restrict__ pos,
+                                                                 const float* __restrict__ dpart, int dks,
+                                                                 int64_t dslice) {
+  __shared__ float red[3][kCtThreads / 64];
+  const int H = A.H, m = blockIdx.x;
+  const bool in = 4 * (int)threadIdx.x < H;
+  const int i = min(4 * (int)threadIdx.x, H - 4);
+  const int64_t o = (int64_t)m * H + i;
+  float4 r[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) r[k] = ld4(down + (int64_t)pos[m * K + k] * H + i);
+  float4 d = ld4(dpart + o);
+  const float4 w1 = ld4(A.post_ffw1 + i), w2 = ld4(A.post_ffw2 + i), wp = ld4(A.post_ffw + i), h = ld4(A.h + o);
+  for (int s = 1; s < dks; ++s) d = fma4(1.f, ld4(dpart + s * dslice + o), d);
+  float4 mo = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < K; ++k) mo = fma4(A.topk_w[m * K + k], r[k], mo);
+  if (in) {
+    *reinterpret_cast<float4*>(A.moe_out + o) = mo;
+    *reinterpret_cast<float4*>(A.dense_out + o) = d;
+  }
+  const float s1 = wave_sum(in ? dot4(d) : 0.f), s2 = wave_sum(in ? dot4(mo) : 0.f);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s1;
+    red[1][threadIdx.x >> 6] = s2;
+  }
+  lds_sync();
+  float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+  for (int w = 0; w < kCtThreads / 64; ++w) {
+    t1 += red[0][w];
+    t2 += red[1][w];
+  }
+  const float i1 = rms_inv(t1, H, A.eps), i2 = rms_inv(t2, H, A.eps);
+  const float4 c = make_float4(d.x * i1 * w1.x + mo.x * i2 * w2.x, d.y * i1 * w1.y + mo.y * i2 * w2.y,
+                               d.z * i1 * w1.z + mo.z * i2 * w2.z, d.w * i1 * w1.w + mo.w * i2 * w2.w);
+  const float i3 = rms_inv(ct_sum(in ? dot4(c) : 0.f, red[2]), H, A.eps);
+  if (in) {
+    const float4 y = make_float4((h.x + c.x * i3 * wp.x) * A.layer_scale, (h.y + c.y * i3 * wp.y) * A.layer_scale,
+                                 (h.z + c.z * i3 * wp.z) * A.layer_scale, (h.w + c.w * i3 * wp.w) * A.layer_scale);
+    __builtin_memcpy(A.h_out + o, &y, 16);
+  }
 }
 
 }  // namespace
@@ -133,9 +205,9 @@ size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* 
 
 int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipStream_t st) {
   const int H = base.H, E = base.E, FF = base.FF, FF2 = base.FF2;
-  if (M < 1 || (int64_t)M * K > 8192)
+  if (M < 1 || M > kMoePfMaxTokens)
     return e4b_fail(E4B_EINVAL, "MoE prefill: %d tokens (1..1024 per call)", M);
-  if (E < K || E > 256 || H % 256 || FF % 32 || FF2 % 32)
+  if (E < K || E > 256 || H % 256 || H > 4 * kCtThreads || FF % 32 || FF2 % 32)
     return e4b_fail(E4B_EINVAL, "MoE prefill: bad shape (H=%d E=%d FF=%d FF2=%d)", H, E, FF, FF2);
   MoeArgs a = base;
   a.scores = b.scores;
@@ -198,8 +270,8 @@ int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipS
   d.ff = 0;
   d.ks = q40_gemm_best_kslices(H, a.dense_down.nb, M, kMoePfDenseKs);
   if ((rc = launch_q40_gemm(d, st))) return rc;
-  hipLaunchKernelGGL(k_moe_combine_rows, dim3((H + 255) / 256, M), dim3(256), 0, st, b.d_sorted, b.pos, b.topk_w, H,
-                     b.moe_out, b.dd_part, d.ks, (int64_t)M * H, b.dense_out);
+  hipLaunchKernelGGL(k_moe_combine_tail, dim3(M), dim3(kCtThreads), 0, st, a, b.d_sorted, b.pos, b.dd_part, d.ks,
+                     (int64_t)M * H);
   E4B_HIP(hipGetLastError());
-  return launch_moe_tail_rows(a, M, st);
+  return E4B_OK;
 }

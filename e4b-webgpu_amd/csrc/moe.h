@@ -50,11 +50,10 @@ int launch_moe_router(const MoeArgs& a, hipStream_t st);
 int launch_moe_topk(const MoeArgs& a, hipStream_t st);
 // the whole half-layer: router, gate/up, down, tail
 int launch_moe_ffn(const MoeArgs& a, hipStream_t st);
-// the same router / top-8 / tail kernels over M token rows (row y of h, xd,
-// xm, dense_out, moe_out, h_out at y * H, of scores at y * E, of topk at y * 8)
+// the router and the top-8 over M token rows (row y of h, xd, xm at y * H, of
+// scores at y * E, of topk at y * 8)
 int launch_moe_router_rows(const MoeArgs& a, int M, hipStream_t st);
 int launch_moe_topk_rows(const MoeArgs& a, int M, hipStream_t st);
-int launch_moe_tail_rows(const MoeArgs& a, int M, hipStream_t st);
 
 // ---- batched prefill of the half-layer (k_moe_prefill.hip) -----------------
 struct MoePrefillBufs {
