@@ -11,5 +11,4 @@ VariantSet variants_f32();      // rows of an even number of blocks
 VariantSet variants_glu();
 VariantSet variants_f32_odd();  // of an odd number
 VariantSet variants_glu_odd();
-VariantSet variants_grp(bool glu, bool aligned);  // grouped: one each
 }  // namespace gemm

@@ -13,10 +13,10 @@ namespace gemm {
 // which some shape lost most)
 VariantSet variants_f32() {
   static const Variant v[] = {
-      GEMM_VARIANT(4, 2, 4, 1, 2, GEMM_F32, false, true, 230), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, false, true, 170),
-      GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, false, true, 108), GEMM_VARIANT(2, 1, 2, 2, 2, GEMM_F32, false, true, 108),
-      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, false, true, 76),  GEMM_VARIANT(1, 1, 2, 2, 2, GEMM_F32, false, true, 76),
-      GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, false, true, 76),
+      GEMM_VARIANT(4, 2, 4, 1, 2, GEMM_F32, true, 230), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, true, 170),
+      GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, true, 108), GEMM_VARIANT(2, 1, 2, 2, 2, GEMM_F32, true, 108),
+      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, true, 76),  GEMM_VARIANT(1, 1, 2, 2, 2, GEMM_F32, true, 76),
+      GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, true, 76),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }
@@ -28,9 +28,8 @@ namespace {
 using gemm::Variant;
 using gemm::VariantSet;
 
-VariantSet variants(int epi, bool grp, bool aligned) {
+VariantSet variants(int epi, bool aligned) {
   using namespace gemm;
-  if (grp) return variants_grp(epi == GEMM_GLU, aligned);
   if (epi == GEMM_GLU) return aligned ? variants_glu() : variants_glu_odd();
   return aligned ? variants_f32() : variants_f32_odd();
 }
@@ -93,7 +92,7 @@ int q40_gemm_kslices(int nb, int want) {
 }
 
 int q40_gemm_best_kslices(int64_t rows, int nb, int M, int most) {
-  const VariantSet s = variants(GEMM_F32, false, nb % 2 == 0);
+  const VariantSet s = variants(GEMM_F32, nb % 2 == 0);
   int best = 1;
   double tb = 0;
   for (int want = 1; want <= most; want *= 2) {
@@ -122,17 +121,13 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
   const int ks = a.ks > 0 ? a.ks : 1;
   if (ks > 1 && a.epi != GEMM_F32) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: split-K needs the f32 epilogue");
   if (ks > W.nb) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d K slices for %d blocks", ks, W.nb);
-  const bool grp = a.tiles != nullptr;
-  if (grp && (!a.ntiles || a.max_tiles < 1 || a.group_rows < 1 || W.rows % a.group_rows || ks != 1 ||
-              (a.gather && a.gather_div < 1)))
-    return e4b_fail(E4B_EINVAL, "q4_0 GEMM: bad grouped-mode arguments");
-  int64_t units = grp ? a.group_rows : W.rows;
+  int64_t units = W.rows;
   switch (a.epi) {
     case GEMM_F32:
       if (!a.Y) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: null output");
       break;
     case GEMM_GLU:
-      if (!a.Yh || a.ff < 1 || 2 * a.ff != (grp ? a.group_rows : W.rows))
+      if (!a.Yh || a.ff < 1 || 2 * a.ff != W.rows)
         return e4b_fail(E4B_EINVAL, "q4_0 GEMM: GeGLU needs 2*ff rows");
       units = a.ff;
       break;
@@ -144,17 +139,13 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
   const int kslices = (W.nb + nbs - 1) / nbs;
   if (kslices != ks)
     return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d blocks do not split into %d slices (use q40_gemm_kslices)", W.nb, ks);
-  const VariantSet set = variants(a.epi, grp, W.nb % 2 == 0);
-  if (!set.n) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d blocks", W.nb);
+  const VariantSet set = variants(a.epi, W.nb % 2 == 0);
   // the kernel addresses activations by 32-bit byte offsets and token tiles
   // by grid y: more tokens than those hold go in several launches
   const int64_t row_bytes = (int64_t)a.ldx * 2;
   int64_t most = (int64_t)0xffffffffll / row_bytes;
   most = std::min<int64_t>(most, 65535 * 32) / 128 * 128;
-  if (grp) {
-    if (a.M > 0xffffffffll / row_bytes) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d grouped rows of %d", a.M, a.ldx);
-    set.v[0].go(a, nbs, (unsigned)a.max_tiles, 1, st);
-  } else if (a.M <= most) {
+  if (a.M <= most) {
     const Variant& v = choose(set, a.epi, units, W.nb, a.M, ks, nullptr);
     v.go(a, nbs, (unsigned)((a.M + 32 * v.T - 1) / (32 * v.T)), (unsigned)ks, st);
   } else {

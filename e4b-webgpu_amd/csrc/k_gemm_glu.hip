@@ -7,9 +7,9 @@ namespace gemm {
 // and 4; 32 x 32, 8 and 4
 VariantSet variants_glu() {
   static const Variant v[] = {
-      GEMM_VARIANT(4, 2, 8, 1, 2, GEMM_GLU, false, true, 230), GEMM_VARIANT(2, 2, 4, 2, 2, GEMM_GLU, false, true, 170),
-      GEMM_VARIANT(2, 2, 2, 4, 2, GEMM_GLU, false, true, 170), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, false, true, 170),
-      GEMM_VARIANT(1, 2, 1, 4, 2, GEMM_GLU, false, true, 110), GEMM_VARIANT(1, 2, 1, 8, 2, GEMM_GLU, false, true, 110),
+      GEMM_VARIANT(4, 2, 8, 1, 2, GEMM_GLU, true, 230), GEMM_VARIANT(2, 2, 4, 2, 2, GEMM_GLU, true, 170),
+      GEMM_VARIANT(2, 2, 2, 4, 2, GEMM_GLU, true, 170), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, true, 170),
+      GEMM_VARIANT(1, 2, 1, 4, 2, GEMM_GLU, true, 110), GEMM_VARIANT(1, 2, 1, 8, 2, GEMM_GLU, true, 110),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }

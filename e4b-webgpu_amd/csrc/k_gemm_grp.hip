@@ -1,20 +1,54 @@
-// k_gemm_grp.hip -- the q4_0 GEMM's grouped variants (the expert-indexed MoE
-// prefill): row tiles of up to 64 draws of one expert.
+// k_gemm_grp.hip -- the q4_0 GEMM's grouped launch (the expert-indexed MoE
+// prefill): row tiles of up to 64 draws of one expert, and beside them the
+// tiles of an ordinary product over all token rows (the dense branch).
+#include "../../include/e4b.h"
 #include "gemm_variants.h"
+#include "util.h"
 
 namespace gemm {
 
-// 64 draws x 64 outputs (GeGLU) or 128 columns (f32), 4 waves.  The GeGLU's
-// rows are the hidden size, a multiple of 256; the down projection's, the
-// expert FFN, may hold an odd number of blocks.
-VariantSet variants_grp(bool glu, bool aligned) {
-  static const Variant v[] = {
-      GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, true, false, 170),
-      GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, true, true, 170),
-      GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, true, true, 170),
-  };
-  if (glu) return {v + 2, aligned ? 1 : 0};
-  return {v + (aligned ? 1 : 0), 1};
+// 64 draws x 64 outputs (GeGLU) or 128 columns (f32), 4 waves.  Rows of an odd
+// number of blocks in either matrix take the kernel that loads scales singly.
+template <int EPI, bool ALN>
+void go_grp(const GemmArgs& g, const GemmArgs& d, hipStream_t st) {
+  constexpr int T = 2, NT = 2, RW = 2, KW = 2, KBL = 2;
+  constexpr int UC = EPI == GEMM_GLU ? 32 * RW : 32 * RW * NT, TOK = 32 * T;
+  static_assert(TOK == kGroupTileRows, "a group's row tile");
+  const int64_t gu = EPI == GEMM_GLU ? g.ff : g.group_rows, du = EPI == GEMM_GLU ? d.ff : d.W.rows;
+  const int gbx = (int)((gu + UC - 1) / UC), dbx = (int)((du + UC - 1) / UC);
+  const int ndense = dbx * ((d.M + TOK - 1) / TOK);
+  hipLaunchKernelGGL((k_q40_gemm_grp<T, NT, RW, KW, KBL, EPI, ALN>), dim3((unsigned)(ndense + gbx * g.max_tiles)),
+                     dim3(64 * RW * KW), 0, st, g, d, ndense, dbx, gbx);
 }
 
 }  // namespace gemm
+
+int launch_q40_gemm_grouped(const GemmArgs& g, const GemmArgs& d, hipStream_t st) {
+  for (const GemmArgs* a : {&g, &d}) {
+    const int K = a->W.nb * 32;
+    if (a->M < 1 || K < 32) return e4b_fail(E4B_EINVAL, "grouped q4_0 GEMM: empty operand (M=%d K=%d)", a->M, K);
+    if ((uint64_t)a->W.rows * (uint64_t)a->W.nb * 16u > 0xffffffffull)
+      return e4b_fail(E4B_EINVAL, "q4_0 GEMM: a %lld x %d-block matrix exceeds the 4 GiB plane limit",
+                      (long long)a->W.rows, a->W.nb);
+    if (a->ldx < K || a->ldx % 8 || a->M > 0xffffffffll / (2 * (int64_t)a->ldx))
+      return e4b_fail(E4B_EINVAL, "grouped q4_0 GEMM: %d rows, stride %d", a->M, a->ldx);
+    if (a->epi != g.epi || (a->epi != GEMM_F32 && a->epi != GEMM_GLU) || a->ks > 1)
+      return e4b_fail(E4B_EINVAL, "grouped q4_0 GEMM: epilogues %d and %d, %d slices", g.epi, d.epi, a->ks);
+    if (a->epi == GEMM_F32 ? !a->Y : (!a->Yh || a->ff < 1 || 2 * a->ff != (a == &g ? g.group_rows : d.W.rows)))
+      return e4b_fail(E4B_EINVAL, "grouped q4_0 GEMM: outputs");
+  }
+  if (!g.tiles || !g.ntiles || g.max_tiles < 1 || g.group_rows < 1 || g.W.rows % g.group_rows ||
+      (g.gather && g.gather_div < 1))
+    return e4b_fail(E4B_EINVAL, "q4_0 GEMM: bad grouped-mode arguments");
+  const bool aligned = g.W.nb % 2 == 0 && d.W.nb % 2 == 0;
+  if (g.epi == GEMM_GLU) {
+    if (!aligned) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d blocks", g.W.nb);
+    gemm::go_grp<GEMM_GLU, true>(g, d, st);
+  } else if (aligned) {
+    gemm::go_grp<GEMM_F32, true>(g, d, st);
+  } else {
+    gemm::go_grp<GEMM_F32, false>(g, d, st);
+  }
+  E4B_HIP(hipGetLastError());
+  return E4B_OK;
+}

@@ -8,11 +8,14 @@
 //   k_moe_group         counting sort of the M*8 (token, slot) draws by expert
 //                       into contiguous runs, cut into tiles of <= 64 rows
 //   grouped GEMMs       expert gate/up + GeGLU and expert down on the matrix
-//                       cores (k_gemm.hip grouped mode): each tile reads its
-//                       expert's rows once for up to 64 draws
-//   dense branch        gate|up + GeGLU GEMM, down GEMM (K slices) over all M tokens
+//                       cores (k_gemm_grp.hip): each tile reads its expert's
+//                       rows once for up to 64 draws; the dense branch's two
+//                       products over all M tokens are tiles of the same
+//                       launches
 //   k_moe_combine_tail  moe[m] = sum_k w_k down_sorted[pos(m, k)], in k order,
-//                       the dense down's K slices summed, and the decode tail
+//                       and the decode tail
+#include <algorithm>
+
 #include "../../include/e4b.h"
 #include "kernels.h"
 #include "moe.h"
@@ -22,7 +25,7 @@ namespace {
 
 constexpr int K = kMoeTopK;
 constexpr int kMoePfMaxTokens = 1024;
-constexpr int kTileRows = 64;  // the grouped GEMM's row tile
+constexpr int kTileRows = kGroupTileRows;
 
 // one workgroup: histogram of the draws' experts in LDS, exclusive scan,
 // placement (list[slot] = draw, pos[draw] = slot) and the tile table.  The
@@ -84,9 +87,8 @@ __global__ __launch_bounds__(1024) void k_moe_group(const uint32_t* __restrict__
 }
 
 // One workgroup per token row m: moe[m] = sum_k w[m][k] down[pos[m K + k]], in
-// slot order, dense[m] = the sum of the dense down GEMM's dks K slices, in
-// slice order, and the decode tail (k_moe_tail) of the two, which stay in
-// registers.  Bounded by the reads of the K sorted rows: a thread owns four
+// slot order, and the decode tail (k_moe_tail) of it and the dense branch's
+// output.  Bounded by the reads of the K sorted rows: a thread owns four
 // adjacent elements, so that all its loads are in flight at once (12 single
 // elements a thread, in a loop, took 22 us over 512 rows).
 // Measured over 512 rows of 2816: 13.4 us, in two kernels 9.9 + 6.6 and the
@@ -111,9 +113,7 @@ DEV float ct_sum(float v, float* red) {  // over the workgroup; red: one float a
   return s;
 }
 __global__ __launch_bounds__(kCtThreads) void k_moe_combine_tail(MoeArgs A, const float* __restrict__ down,
-                                                                 const uint32_t* __restrict__ pos,
-                                                                 const float* __restrict__ dpart, int dks,
-                                                                 int64_t dslice) {
+                                                                 const uint32_t* __restrict__ pos) {
   __shared__ float red[3][kCtThreads / 64];
   const int H = A.H, m = blockIdx.x;
   const bool in = 4 * (int)threadIdx.x < H;
@@ -122,16 +122,12 @@ __global__ __launch_bounds__(kCtThreads) void k_moe_combine_tail(MoeArgs A, cons
   float4 r[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) r[k] = ld4(down + (int64_t)pos[m * K + k] * H + i);
-  float4 d = ld4(dpart + o);
+  const float4 d = ld4(A.dense_out + o);
   const float4 w1 = ld4(A.post_ffw1 + i), w2 = ld4(A.post_ffw2 + i), wp = ld4(A.post_ffw + i), h = ld4(A.h + o);
-  for (int s = 1; s < dks; ++s) d = fma4(1.f, ld4(dpart + s * dslice + o), d);
   float4 mo = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int k = 0; k < K; ++k) mo = fma4(A.topk_w[m * K + k], r[k], mo);
-  if (in) {
-    *reinterpret_cast<float4*>(A.moe_out + o) = mo;
-    *reinterpret_cast<float4*>(A.dense_out + o) = d;
-  }
+  if (in) *reinterpret_cast<float4*>(A.moe_out + o) = mo;
   const float s1 = wave_sum(in ? dot4(d) : 0.f), s2 = wave_sum(in ? dot4(mo) : 0.f);
   if ((threadIdx.x & 63) == 0) {
     red[0][threadIdx.x >> 6] = s1;
@@ -160,7 +156,8 @@ __global__ __launch_bounds__(kCtThreads) void k_moe_combine_tail(MoeArgs A, cons
 size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* base) {
   const int H = a.H, E = a.E, FF = a.FF, FF2 = a.FF2;
   const size_t P = (size_t)M * K;
-  const int max_tiles = E + (int)((P + kTileRows - 1) / kTileRows);
+  // the most tiles: every expert that P draws can reach ends in a part-empty one
+  const int max_tiles = (int)((P + (kTileRows - 1) * std::min<size_t>(E, P)) / kTileRows);
   size_t cur = 0;
   auto take = [&](size_t bytes) {
     uint8_t* p = base ? base + cur : nullptr;
@@ -179,7 +176,6 @@ size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* 
   uint8_t* p_g = take(P * FF * 2);
   uint8_t* p_d = take(P * H * 4);
   uint8_t* p_gd = take((size_t)M * FF2 * 2);
-  uint8_t* p_ddp = take((size_t)kMoePfDenseKs * M * H * 4);
   uint8_t* p_dense = take((size_t)M * H * 4);
   uint8_t* p_moe = take((size_t)M * H * 4);
   if (b) {
@@ -196,7 +192,6 @@ size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* 
     b->g_sorted = (uint16_t*)p_g;
     b->d_sorted = (float*)p_d;
     b->g_dense = (uint16_t*)p_gd;
-    b->dd_part = (float*)p_ddp;
     b->dense_out = (float*)p_dense;
     b->moe_out = (float*)p_moe;
   }
@@ -221,8 +216,9 @@ int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipS
   if ((rc = launch_moe_router_rows(a, M, st)) || (rc = launch_moe_topk_rows(a, M, st))) return rc;
   hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(1024), 0, st, b.topk_idx, M * K, E, b.list, b.pos, b.tiles, b.ntiles);
   E4B_HIP(hipGetLastError());
-  // expert gate/up + GeGLU over the sorted draws, then expert down
-  GemmArgs g{};
+  // expert gate/up + GeGLU over the sorted draws and the dense branch's over
+  // all tokens in one launch, then both down projections in another
+  GemmArgs g{}, d{};
   g.W = a.exp_gu;
   g.X = b.xm;
   g.M = M * K;
@@ -237,7 +233,15 @@ int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipS
   g.group_rows = 2 * (int64_t)FF;
   g.gather = b.list;
   g.gather_div = K;
-  if ((rc = launch_q40_gemm(g, st))) return rc;
+  d.W = a.dense_gu;
+  d.X = b.xd;
+  d.M = M;
+  d.ldx = H;
+  d.epi = GEMM_GLU;
+  d.Yh = b.g_dense;
+  d.ff = FF2;
+  d.ks = 1;
+  if ((rc = launch_q40_gemm_grouped(g, d, st))) return rc;
   g.W = a.exp_down;
   g.X = b.g_sorted;
   g.ldx = FF;
@@ -248,30 +252,15 @@ int launch_moe_prefill(const MoeArgs& base, int M, const MoePrefillBufs& b, hipS
   g.group_rows = H;
   g.gather = nullptr;
   g.gather_div = 1;
-  if ((rc = launch_q40_gemm(g, st))) return rc;
-  // dense branch over all tokens; the down projection's K slices are summed
-  // by the combine
-  GemmArgs d{};
-  d.W = a.dense_gu;
-  d.X = b.xd;
-  d.M = M;
-  d.ldx = H;
-  d.epi = GEMM_GLU;
-  d.Yh = b.g_dense;
-  d.ff = FF2;
-  d.ks = 1;
-  if ((rc = launch_q40_gemm(d, st))) return rc;
   d.W = a.dense_down;
   d.X = b.g_dense;
   d.ldx = FF2;
   d.epi = GEMM_F32;
-  d.Y = b.dd_part;
+  d.Y = a.dense_out;
   d.Yh = nullptr;
   d.ff = 0;
-  d.ks = q40_gemm_best_kslices(H, a.dense_down.nb, M, kMoePfDenseKs);
-  if ((rc = launch_q40_gemm(d, st))) return rc;
-  hipLaunchKernelGGL(k_moe_combine_tail, dim3(M), dim3(kCtThreads), 0, st, a, b.d_sorted, b.pos, b.dd_part, d.ks,
-                     (int64_t)M * H);
+  if ((rc = launch_q40_gemm_grouped(g, d, st))) return rc;
+  hipLaunchKernelGGL(k_moe_combine_tail, dim3(M), dim3(kCtThreads), 0, st, a, b.d_sorted, b.pos);
   E4B_HIP(hipGetLastError());
   return E4B_OK;
 }

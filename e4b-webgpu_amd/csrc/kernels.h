@@ -129,9 +129,9 @@ struct GemmArgs {
   uint16_t* Yh;
   int64_t ff;
   int ks;             // split-K slices (GEMM_F32)
-  // grouped mode (the expert-indexed MoE prefill; tiles != null): blockIdx.y
-  // picks tiles[y] = (group g, first row r0, rows n <= 64) of the M sorted
-  // rows, y < *ntiles; the weights are rows [g group_rows, (g+1) group_rows)
+  // launch_q40_gemm_grouped only (the expert-indexed MoE prefill): tiles[y] =
+  // (group g, first row r0, rows n <= kGroupTileRows) of the M sorted rows,
+  // y < *ntiles <= max_tiles; the weights are rows [g group_rows, (g+1) group_rows)
   // of W (GLU: group_rows = 2 ff, gate then up); X row r is gather[r] /
   // gather_div (gather null: row r); outputs are rows r0 .. r0 + n - 1 of an
   // [M][group_rows] (GLU: [M][ff]) matrix
@@ -143,6 +143,10 @@ struct GemmArgs {
   int gather_div;
 };
 int launch_q40_gemm(const GemmArgs& a, hipStream_t st);
+constexpr int kGroupTileRows = 64;
+// a grouped product and an ordinary one (of the same epilogue, one K slice)
+// in one launch
+int launch_q40_gemm_grouped(const GemmArgs& grouped, const GemmArgs& dense, hipStream_t st);
 // the largest split-K slice count <= want that cuts nb blocks into whole
 // slices (what GemmArgs::ks must be)
 int q40_gemm_kslices(int nb, int want);

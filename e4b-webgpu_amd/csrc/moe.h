@@ -69,13 +69,9 @@ struct MoePrefillBufs {
   uint16_t* g_sorted;  // [M*8][FF] f16 expert GeGLU outputs, sorted
   float* d_sorted;     // [M*8][H] expert down outputs, sorted
   uint16_t* g_dense;   // [M][FF2]
-  float* dd_part;      // [kMoePfDenseKs][M][H] dense down split-K partials
   float* dense_out;    // [M][H]
   float* moe_out;      // [M][H]
 };
-// the most K slices of the dense down GEMM over the prompt rows (the combine
-// sums them)
-constexpr int kMoePfDenseKs = 2;
 // bytes of scratch for M tokens; with base != null also fills b from it
 size_t moe_prefill_scratch(const MoeArgs& a, int M, MoePrefillBufs* b, uint8_t* base);
 // h_out[m] (a.h_out, rows of H) for the M token rows of a.h
