@@ -70,11 +70,13 @@ DEV h8 nib_word_f16(uint32_t w, uint32_t mag) {
 }
 
 // gelu_tanh (common.h) as g / (1 + e^-2t): 1 + tanh(t) = 2 / (1 + e^-2t), a
-// dozen instructions instead of tanhf's fifty, and no cancellation for t < 0
+// dozen instructions instead of tanhf's fifty, and no cancellation for t < 0.
+// At the clamp, t <= -20, it is 0 as there (tanhf(-20) is -1): e^-40 g would
+// grow with a large gate again.
 DEV float gelu_sigmoid(float g) {
-  float t = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-  t = fminf(fmaxf(t, -20.f), 20.f);
-  return g / (1.f + __expf(-2.f * t));
+  const float t = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+  const float e = t > -20.f ? __expf(-2.f * fminf(t, 20.f)) : __builtin_inff();
+  return g / (1.f + e);
 }
 
 __device__ const uint4 kZeros[8] = {};
