@@ -144,12 +144,13 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
   // by grid y: more tokens than those hold go in several launches
   const int64_t row_bytes = (int64_t)a.ldx * 2;
   int64_t most = (int64_t)0xffffffffll / row_bytes;
-  most = std::min<int64_t>(most, 65535 * 32) / 128 * 128;
+  most = std::min<int64_t>(most, 65535 * 32);
+  if (most >= 128) most = most / 128 * 128;  // whole tiles (rows of 32 MiB and more: as many as fit)
   if (a.M <= most) {
     const Variant& v = choose(set, a.epi, units, W.nb, a.M, ks, nullptr);
     v.go(a, nbs, (unsigned)((a.M + 32 * v.T - 1) / (32 * v.T)), (unsigned)ks, st);
   } else {
-    if (ks > 1 || most < 1) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d rows of %d in %d K slices", a.M, a.ldx, ks);
+    if (ks > 1) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d rows of %d in %d K slices", a.M, a.ldx, ks);
     for (int64_t m0 = 0; m0 < a.M; m0 += most) {
       GemmArgs c = a;
       c.M = (int)std::min<int64_t>(most, a.M - m0);
