@@ -38,6 +38,7 @@
 // us, 3072 x 2048 over 37 tokens 17.7 -> 5 us (MI355X; before: 4 waves, one
 // K group, operands staged through registers).
 #pragma once
+#include <atomic>
 #include <type_traits>
 
 #include "kernels.h"
@@ -448,10 +449,13 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_q40_gemm_grp(GemmArgs g, Ge
 }
 
 // The variants k_gemm.hip chooses from; each translation unit instantiates
-// its own.  A variant's launcher.
+// its own.  A variant's kernel and launcher, and how many of its workgroups
+// share a CU (0: not asked for yet).
 struct Variant {
-  int T, NT, RW, KW, KBL, lds, vgprs;
+  int T, NT, RW, KW, KBL;
+  const void* kernel;
   void (*go)(const GemmArgs& a, int ks_blocks, unsigned gy, unsigned gz, hipStream_t st);
+  std::atomic<int> occ{0};
 };
 
 template <int T, int NT, int RW, int KW, int KBL, int EPI, bool ALN>
@@ -463,11 +467,10 @@ void launch_variant(const GemmArgs& a, int nbs, unsigned gy, unsigned gz, hipStr
                      dim3(S::NTHR), 0, st, a, a.W.nb, nbs);
 }
 
-#define GEMM_VARIANT(T, NT, RW, KW, KBL, EPI, ALN, VGPRS)                                           \
-  {                                                                                                 \
-    T, NT, RW, KW, KBL,                                                                             \
-        2 * Shape<T, NT, RW, KW, KBL>::BUF * 16 + Shape<T, NT, RW, KW, KBL>::COLS * KW * KBL * 4,   \
-        VGPRS, launch_variant<T, NT, RW, KW, KBL, EPI, ALN>                                         \
+#define GEMM_VARIANT(T, NT, RW, KW, KBL, EPI, ALN)                                                   \
+  {                                                                                                  \
+    T, NT, RW, KW, KBL, reinterpret_cast<const void*>(k_q40_gemm<T, NT, RW, KW, KBL, EPI, ALN>),     \
+        launch_variant<T, NT, RW, KW, KBL, EPI, ALN>                                                 \
   }
 
 }  // namespace gemm

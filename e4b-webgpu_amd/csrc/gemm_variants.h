@@ -4,7 +4,7 @@
 
 namespace gemm {
 struct VariantSet {
-  const Variant* v;
+  Variant* v;
   int n;
 };
 VariantSet variants_f32();      // rows of an even number of blocks

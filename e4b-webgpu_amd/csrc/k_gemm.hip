@@ -1,4 +1,6 @@
 // k_gemm.hip -- choice and launch of the q4_0 GEMM variants (gemm_kernel.h).
+#include <limits.h>
+
 #include <algorithm>
 
 #include "../../include/e4b.h"
@@ -12,11 +14,11 @@ namespace gemm {
 // and 4; 32 x 64, 8 and 4; 32 x 32, 8 (of twelve measured, the seven without
 // which some shape lost most)
 VariantSet variants_f32() {
-  static const Variant v[] = {
-      GEMM_VARIANT(4, 2, 4, 1, 2, GEMM_F32, true, 230), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, true, 170),
-      GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, true, 108), GEMM_VARIANT(2, 1, 2, 2, 2, GEMM_F32, true, 108),
-      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, true, 76),  GEMM_VARIANT(1, 1, 2, 2, 2, GEMM_F32, true, 76),
-      GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, true, 76),
+  static Variant v[] = {
+      GEMM_VARIANT(4, 2, 4, 1, 2, GEMM_F32, true), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, true),
+      GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, true), GEMM_VARIANT(2, 1, 2, 2, 2, GEMM_F32, true),
+      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, true), GEMM_VARIANT(1, 1, 2, 2, 2, GEMM_F32, true),
+      GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, true),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }
@@ -40,40 +42,61 @@ VariantSet variants(int epi, bool aligned) {
 // are compared by this model instead of by thresholds.  A stage of one
 // workgroup takes at least its latency (copies, barrier, the waves' chain of
 // dependent matrix instructions); the workgroups that share a CU add up their
-// work: 32 x 32 x 32 units at 111 / 82 / 63 ns of a SIMD for 1 / 2 / 4 token
+// work: 32 x 32 x 32 units at 107 / 81 / 65 ns of a SIMD for 1 / 2 / 4 token
 // tiles a wave (the nibble conversion is shared by them).  Constants fitted
-// on MI355X to 1000 timings of 12 variants (256..32768 rows, 256..16384
-// columns, 1..512 tokens): 10 % rms; the variant it picks is 1.4 % slower
-// than the best on average, 22 % at worst.
-double gemm_cost_us(const Variant& v, int epi, int64_t units, int nb, int64_t M, int ks) {
+// on MI355X to the times of all variants over 3000 shapes (37..32768 rows,
+// 64..16384 columns, 1..512 tokens), weights in cache and cold.  Over 2000
+// other shapes it is 12 and 14 % rms off, and the variant it picks is 0.4 %
+// slower than the best on average, 30 % at worst.
+// Eight K groups count as one workgroup a CU also where two fit (rows of an
+// odd number of blocks): two side by side take as long as one after the other
+// (1.23 against 0.61 us a stage).
+double gemm_cost_us(const Variant& v, int resident, int epi, int64_t units, int nb, int64_t M, int ks) {
+  const int occ = v.KW == 8 ? 1 : resident;
   const int waves = v.RW * v.KW, sb = v.KW * v.KBL;
   const int uc = epi == GEMM_GLU ? 32 * v.RW : 32 * v.RW * v.NT;
   const double wgs = (double)((units + uc - 1) / uc) * (double)((M + 32 * v.T - 1) / (32 * v.T)) * ks;
   const double stages = (double)((nb + ks * sb - 1) / (ks * sb));
-  const int by_lds = 163840 / v.lds, by_reg = 4 * (512 / ((v.vgprs + 7) / 8 * 8)) / waves;
-  const int occ = std::max(1, std::min(by_lds, by_reg));
-  const double unit = (v.T == 1 ? 0.111 : v.T == 2 ? 0.082 : 0.0626) / 4;
-  const double lat = 0.289 + 0.061 * v.T * v.NT * v.KBL * std::max(1.0, waves / 4.0);
+  const double unit = (v.T == 1 ? 0.107 : v.T == 2 ? 0.081 : 0.065) / 4;
+  const double lat = 0.373 + 0.047 * v.T * v.NT * v.KBL * std::max(1.0, waves / 4.0);
   const double thr = v.T * v.NT * v.RW * v.KW * v.KBL * unit;
   const double per = (double)(int64_t)((wgs + 255) / 256);  // workgroups of the fullest CU
   const double full = (double)(int64_t)(per / occ), rem = per - full * occ;
   double t = full * std::max(lat, thr * occ) + (rem > 0 ? std::max(lat, thr * rem) : 0.0);
-  t = 2.0 + stages * t + 0.356 * v.T * v.NT * (v.KW == 1 ? 1 : 2) * (full + (rem > 0 ? 1 : 0));
+  t = 1.7 + stages * t + 0.3 * v.T * v.NT * (v.KW == 1 ? 1 : 2) * (full + (rem > 0 ? 1 : 0));
   return t;
 }
 
-const Variant& choose(const VariantSet& s, int epi, int64_t units, int nb, int64_t M, int ks, double* us) {
-  int best = 0;
+// Workgroups of a variant that share a CU, as its kernel was compiled (LDS and
+// registers); the runtime is asked once a variant.  0 and an error message if
+// it does not know the kernel.
+int occupancy(Variant& v) {
+  int occ = v.occ.load(std::memory_order_relaxed);
+  if (occ > 0) return occ;
+  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, v.kernel, 64 * v.RW * v.KW, 0);
+  if (e != hipSuccess || occ < 1) {
+    (void)e4b_fail(E4B_EHIP, "q4_0 GEMM: occupancy of a kernel -> %s", hipGetErrorString(e));
+    return 0;
+  }
+  v.occ.store(occ, std::memory_order_relaxed);
+  return occ;
+}
+
+// the variant of the least estimated time (its estimate in *us), or null
+const Variant* choose(const VariantSet& s, int epi, int64_t units, int nb, int64_t M, int ks, double* us) {
+  const Variant* best = nullptr;
   double tb = 0;
   for (int i = 0; i < s.n; ++i) {
-    const double t = gemm_cost_us(s.v[i], epi, units, nb, M, ks);
-    if (i == 0 || t < tb) {
-      best = i;
+    const int occ = occupancy(s.v[i]);
+    if (!occ) return nullptr;
+    const double t = gemm_cost_us(s.v[i], occ, epi, units, nb, M, ks);
+    if (!best || t < tb) {
+      best = &s.v[i];
       tb = t;
     }
   }
   if (us) *us = tb;
-  return s.v[best];
+  return best;
 }
 
 // q4_0 blocks of a split-K slice: whole pairs of blocks, and the slices of
@@ -97,8 +120,8 @@ int q40_gemm_best_kslices(int64_t rows, int nb, int M, int most) {
   double tb = 0;
   for (int want = 1; want <= most; want *= 2) {
     const int ks = q40_gemm_kslices(nb, want);
-    double t;
-    (void)choose(s, GEMM_F32, rows, nb, M, ks, &t);
+    double t = 0;
+    if (!choose(s, GEMM_F32, rows, nb, M, ks, &t)) return 1;  // (the launch says why)
     // each further slice is written once and read once by the consumer, at
     // about 4 MB a microsecond
     t += (double)(ks - 1) * (double)M * (double)rows * 8.0 / 4e6;
@@ -147,8 +170,9 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
   most = std::min<int64_t>(most, 65535 * 32);
   if (most >= 128) most = most / 128 * 128;  // whole tiles (rows of 32 MiB and more: as many as fit)
   if (a.M <= most) {
-    const Variant& v = choose(set, a.epi, units, W.nb, a.M, ks, nullptr);
-    v.go(a, nbs, (unsigned)((a.M + 32 * v.T - 1) / (32 * v.T)), (unsigned)ks, st);
+    const Variant* v = choose(set, a.epi, units, W.nb, a.M, ks, nullptr);
+    if (!v) return E4B_EHIP;
+    v->go(a, nbs, (unsigned)((a.M + 32 * v->T - 1) / (32 * v->T)), (unsigned)ks, st);
   } else {
     if (ks > 1) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: %d rows of %d in %d K slices", a.M, a.ldx, ks);
     for (int64_t m0 = 0; m0 < a.M; m0 += most) {
@@ -157,8 +181,9 @@ int launch_q40_gemm(const GemmArgs& a, hipStream_t st) {
       c.X = a.X + m0 * a.ldx;
       if (a.Y) c.Y = a.Y + m0 * units;
       if (a.Yh) c.Yh = a.Yh + m0 * units;
-      const Variant& v = choose(set, c.epi, units, W.nb, c.M, 1, nullptr);
-      v.go(c, nbs, (unsigned)((c.M + 32 * v.T - 1) / (32 * v.T)), 1, st);
+      const Variant* v = choose(set, c.epi, units, W.nb, c.M, 1, nullptr);
+      if (!v) return E4B_EHIP;
+      v->go(c, nbs, (unsigned)((c.M + 32 * v->T - 1) / (32 * v->T)), 1, st);
     }
   }
   E4B_HIP(hipGetLastError());
@@ -177,4 +202,23 @@ int launch_q40_gemm(const Q40Mat& W, const uint16_t* X, int M, float* Y, uint16_
   a.ff = ff;
   a.ks = 1;
   return launch_q40_gemm(a, st);
+}
+
+// For the tests of every tile: the one that e4b_k_q40_gemm (geglu 0; units
+// rows) or e4b_k_q40_gemm_geglu (geglu 1; units = ff) takes.  tile: token
+// rows, outputs and waves of a workgroup, K groups, blocks a K stage,
+// workgroups that share a CU.
+extern "C" int e4b_q40_gemm_tile(int64_t units, int64_t cols, int m, int geglu, int32_t* tile) {
+  if (units < 1 || cols < 32 || cols % 32 || cols > INT_MAX || m < 1 || !tile)
+    return e4b_fail(E4B_EINVAL, "e4b_q40_gemm_tile: bad arguments");
+  const int epi = geglu ? GEMM_GLU : GEMM_F32, nb = (int)(cols / 32);
+  const Variant* v = choose(variants(epi, nb % 2 == 0), epi, units, nb, m, 1, nullptr);
+  if (!v) return E4B_EHIP;
+  tile[0] = 32 * v->T;
+  tile[1] = 32 * v->RW * (geglu ? 1 : v->NT);
+  tile[2] = v->RW * v->KW;
+  tile[3] = v->KW;
+  tile[4] = v->KW * v->KBL;
+  tile[5] = v->occ.load(std::memory_order_relaxed);
+  return E4B_OK;
 }

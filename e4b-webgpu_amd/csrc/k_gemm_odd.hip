@@ -6,17 +6,17 @@
 namespace gemm {
 
 VariantSet variants_f32_odd() {
-  static const Variant v[] = {
-      GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, false, 170), GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, false, 108),
-      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, false, 76),  GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, false, 76),
+  static Variant v[] = {
+      GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_F32, false), GEMM_VARIANT(2, 1, 2, 4, 2, GEMM_F32, false),
+      GEMM_VARIANT(1, 1, 2, 4, 2, GEMM_F32, false),  GEMM_VARIANT(1, 1, 1, 8, 2, GEMM_F32, false),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }
 
 VariantSet variants_glu_odd() {
-  static const Variant v[] = {
-      GEMM_VARIANT(2, 2, 4, 2, 2, GEMM_GLU, false, 170), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, false, 170),
-      GEMM_VARIANT(1, 2, 1, 4, 2, GEMM_GLU, false, 110),
+  static Variant v[] = {
+      GEMM_VARIANT(2, 2, 4, 2, 2, GEMM_GLU, false), GEMM_VARIANT(2, 2, 2, 2, 2, GEMM_GLU, false),
+      GEMM_VARIANT(1, 2, 1, 4, 2, GEMM_GLU, false),
   };
   return {v, (int)(sizeof(v) / sizeof(v[0]))};
 }

@@ -8,11 +8,14 @@ that is not full.  Products are exact and sums are f32, so outputs lie within
 1e-5 of max|Y| (2048 columns: f32 rounding of partial sums, 64 blocks x 2^-24,
 is 4e-6 at worst); the GeGLU adds one f16 rounding (2^-11) of the output.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle as orc
 from e4b import formats
+from e4b._lib import check, lib
 from e4b.kernels import MoeLayer, Q40Matrix
 from tests.util import max_rel_err
 
@@ -32,6 +35,22 @@ F32 = [(9176, 192, 639), (14280, 704, 217), (8591, 2048, 35), (14338, 384, 161),
        (61, 384, 5), (5306, 224, 689), (5696, 2016, 65), (151, 224, 2), (312, 288, 1), (33, 64, 33), (1, 32, 1)]
 GLU = [(6717, 192, 326), (6946, 192, 165), (6714, 192, 105), (6569, 384, 97), (76, 192, 2), (152, 384, 1),
        (8744, 224, 139), (6557, 224, 100), (19, 224, 8), (33, 64, 33)]
+
+
+def _tile(outputs, cols, m, geglu):
+    t = (ctypes.c_int32 * 6)()
+    check(lib.e4b_q40_gemm_tile(ctypes.c_int64(outputs), ctypes.c_int64(cols), m, int(geglu), t), "e4b_q40_gemm_tile")
+    return list(t)
+
+
+def test_workgroups_per_cu():
+    # as the kernels were compiled: 160 KB of LDS hold three tiles of 64 x 128
+    # (50 KB; 162 registers allow three waves a SIMD), and of the tile of
+    # eight K groups two where rows have an odd number of blocks (no staged
+    # scales: 80 KB), else one
+    assert _tile(10890, 448, 260, False)[:1] + _tile(10890, 448, 260, False)[5:] == [64, 3]
+    assert _tile(33, 288, 1, False)[3:] == [8, 16, 2]
+    assert _tile(33, 320, 1, False)[3:] == [8, 16, 1]
 
 
 @pytest.mark.parametrize("rows,cols,m", F32)
