@@ -2,9 +2,11 @@
 its tiles, against float64 products of the same f16 activations and the
 oracle's dequantised weights.
 
-The variant follows from the shape (rows, columns, tokens); the first lists
-hold one shape for each, all ragged in rows and tokens and with a last K stage
-that is not full.  Products are exact and sums are f32, so outputs lie within
+The variant follows from the shape (rows, columns, tokens).  The lists hold,
+for each, a shape that is ragged in rows and in tokens and ends in a K stage
+that is not full (a stage of two blocks over rows of an even number always
+is); test_lists_hold_every_tile asks the library for the choices and checks
+that.  Products are exact and sums are f32, so outputs lie within
 1e-5 of max|Y| (2048 columns: f32 rounding of partial sums, 64 blocks x 2^-24,
 is 4e-6 at worst); the GeGLU adds one f16 rounding (2^-11) of the output.
 """
@@ -30,17 +32,42 @@ def _gelu(g):
     return 0.5 * g * (1 + np.tanh(np.clip(0.7978845608028654 * (g + 0.044715 * g ** 3), -20, 20)))
 
 
-# rows of an even number of blocks (64 x 3 .. 2048), then of an odd number
+# rows of an even number of blocks (64 x 1 .. 2048), then of an odd number
 F32 = [(9176, 192, 639), (14280, 704, 217), (8591, 2048, 35), (14338, 384, 161), (102, 192, 3), (17554, 384, 1),
-       (61, 384, 5), (5306, 224, 689), (5696, 2016, 65), (151, 224, 2), (312, 288, 1), (33, 64, 33), (1, 32, 1)]
+       (18046, 64, 294), (10890, 448, 260), (5833, 1600, 67), (12647, 448, 99), (8234, 192, 1), (16425, 64, 1),
+       (33, 320, 1),
+       (61, 384, 5), (5306, 224, 689), (5696, 2016, 65), (151, 224, 2), (312, 288, 1), (33, 64, 33), (1, 32, 1),
+       (16947, 96, 162), (12724, 96, 98), (8206, 96, 1), (33, 288, 1)]
 GLU = [(6717, 192, 326), (6946, 192, 165), (6714, 192, 105), (6569, 384, 97), (76, 192, 2), (152, 384, 1),
-       (8744, 224, 139), (6557, 224, 100), (19, 224, 8), (33, 64, 33)]
+       (17266, 64, 130), (16388, 320, 129), (6281, 192, 104), (6382, 64, 99), (33, 64, 1), (33, 320, 1),
+       (8744, 224, 139), (6557, 224, 100), (19, 224, 8), (33, 64, 33),
+       (19705, 160, 136), (6176, 96, 97), (33, 96, 1)]
+# token rows, outputs, waves and K groups of the tiles, for rows of an even
+# and of an odd number of blocks
+TILES = {(False, False): {(128, 256, 4, 1), (64, 128, 4, 2), (64, 64, 8, 4), (64, 64, 4, 2), (32, 64, 8, 4),
+                          (32, 64, 4, 2), (32, 32, 8, 8)},
+         (False, True): {(64, 128, 4, 2), (64, 64, 8, 4), (32, 64, 8, 4), (32, 32, 8, 8)},
+         (True, False): {(128, 256, 8, 1), (64, 128, 8, 2), (64, 64, 8, 4), (64, 64, 4, 2), (32, 32, 4, 4),
+                         (32, 32, 8, 8)},
+         (True, True): {(64, 128, 8, 2), (64, 64, 4, 2), (32, 32, 4, 4)}}
 
 
 def _tile(outputs, cols, m, geglu):
     t = (ctypes.c_int32 * 6)()
     check(lib.e4b_q40_gemm_tile(ctypes.c_int64(outputs), ctypes.c_int64(cols), m, int(geglu), t), "e4b_q40_gemm_tile")
     return list(t)
+
+
+@pytest.mark.parametrize("geglu", [False, True])
+def test_lists_hold_every_tile(geglu):
+    seen = {False: set(), True: set()}
+    for outputs, cols, m in GLU if geglu else F32:
+        nb = cols // 32
+        tok, out, waves, kg, stage, _ = _tile(outputs, cols, m, geglu)
+        if outputs % out and m % tok and (nb % stage or (stage == 2 and nb % 2 == 0)):
+            seen[nb % 2 == 1].add((tok, out, waves, kg))
+    for odd in (False, True):
+        assert seen[odd] == TILES[geglu, odd], f"rows of an {'odd' if odd else 'even'} number of blocks"
 
 
 def test_workgroups_per_cu():
