@@ -419,33 +419,35 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_q40_gemm(GemmArgs a, int nb
 }
 
 // A grouped product and an ordinary one in one launch: the first ndense
-// workgroups are tiles of d (dbx of them side by side), the rest of g.  The
-// dense branch of an MoE layer alone leaves most of the chip idle; in front of
-// the experts' tiles it fills the workgroup slots that their last, part-empty
-// wave leaves: a half-layer over 512
-// tokens 247 -> 239 us (MI355X; the dense branch in launches of its own: 30 +
-// 17 us).
-template <int T, int NT, int RW, int KW, int KBL, int EPI, bool ALN>
+// workgroups are tiles of d (dbx of them side by side), the rest of g.  The dense branch of an MoE layer alone leaves most of the
+// chip idle; in front of the experts' tiles it fills the workgroup slots that
+// their last, part-empty wave leaves: a half-layer over 512 tokens 247 -> 239
+// us (MI355X; the dense branch in launches of its own: 30 + 17 us).
+//
+// An expert's last rows often fit one token tile: half the work of two.
+// GALN, DALN: whether g's and d's rows have an even number of blocks, each for
+// its own tiles: a dense width of an odd number must not put the experts'
+// product, the far larger one, on the kernel that loads scales singly.
+template <int T, int NT, int RW, int KW, int KBL, int EPI, bool GALN, bool DALN>
 __global__ __launch_bounds__(64 * RW * KW, 2) void k_q40_gemm_grp(GemmArgs g, GemmArgs d, int ndense, int dbx,
                                                                   int gbx) {
   using S = Shape<T, NT, RW, KW, KBL>;
   __shared__ __align__(16) u32x4 bufa[S::BUF];
   __shared__ __align__(16) u32x4 bufb[S::BUF];
-  __shared__ __align__(16) uint32_t scb[ALN ? S::COLS * S::SB : 4];
+  __shared__ __align__(16) uint32_t scb[GALN || DALN ? S::COLS * S::SB : 4];
   int id = blockIdx.x;
   if (id < ndense) {
     const int by = id / dbx, bx = id % dbx;
-    gemm_tile<T, NT, RW, KW, KBL, EPI, false, ALN>(d, d.W.nb, d.W.nb, bx, by, bufa, bufb, scb);
+    gemm_tile<T, NT, RW, KW, KBL, EPI, false, DALN>(d, d.W.nb, d.W.nb, bx, by, bufa, bufb, scb);
     return;
   }
   id -= ndense;
   const int by = id / gbx, bx = id % gbx;
   if (by >= *g.ntiles) return;  // the grid is sized for the most tiles
-  // an expert's last rows often fit one token tile: half the work of two
   if (T == 2 && g.tiles[by].z <= 32)
-    gemm_tile<1, NT, RW, KW, KBL, EPI, true, ALN>(g, g.W.nb, g.W.nb, bx, by, bufa, bufb, scb);
+    gemm_tile<1, NT, RW, KW, KBL, EPI, true, GALN>(g, g.W.nb, g.W.nb, bx, by, bufa, bufb, scb);
   else
-    gemm_tile<T, NT, RW, KW, KBL, EPI, true, ALN>(g, g.W.nb, g.W.nb, bx, by, bufa, bufb, scb);
+    gemm_tile<T, NT, RW, KW, KBL, EPI, true, GALN>(g, g.W.nb, g.W.nb, bx, by, bufa, bufb, scb);
 }
 
 // The variants k_gemm.hip chooses from; each translation unit instantiates

@@ -7,9 +7,9 @@
 
 namespace gemm {
 
-// 64 draws x 64 outputs (GeGLU) or 128 columns (f32), 4 waves.  Rows of an odd
-// number of blocks in either matrix take the kernel that loads scales singly.
-template <int EPI, bool ALN>
+// 64 draws x 64 outputs (GeGLU) or 128 columns (f32), 4 waves.  A matrix whose
+// rows have an odd number of blocks loads its scales singly, the other not.
+template <int EPI, bool GALN, bool DALN>
 void go_grp(const GemmArgs& g, const GemmArgs& d, hipStream_t st) {
   constexpr int T = 2, NT = 2, RW = 2, KW = 2, KBL = 2;
   constexpr int UC = EPI == GEMM_GLU ? 32 * RW : 32 * RW * NT, TOK = 32 * T;
@@ -17,7 +17,7 @@ void go_grp(const GemmArgs& g, const GemmArgs& d, hipStream_t st) {
   const int64_t gu = EPI == GEMM_GLU ? g.ff : g.group_rows, du = EPI == GEMM_GLU ? d.ff : d.W.rows;
   const int gbx = (int)((gu + UC - 1) / UC), dbx = (int)((du + UC - 1) / UC);
   const int ndense = dbx * ((d.M + TOK - 1) / TOK);
-  hipLaunchKernelGGL((k_q40_gemm_grp<T, NT, RW, KW, KBL, EPI, ALN>), dim3((unsigned)(ndense + gbx * g.max_tiles)),
+  hipLaunchKernelGGL((k_q40_gemm_grp<T, NT, RW, KW, KBL, EPI, GALN, DALN>), dim3((unsigned)(ndense + gbx * g.max_tiles)),
                      dim3(64 * RW * KW), 0, st, g, d, ndense, dbx, gbx);
 }
 
@@ -40,14 +40,13 @@ int launch_q40_gemm_grouped(const GemmArgs& g, const GemmArgs& d, hipStream_t st
   if (!g.tiles || !g.ntiles || g.max_tiles < 1 || g.group_rows < 1 || g.W.rows % g.group_rows ||
       (g.gather && g.gather_div < 1))
     return e4b_fail(E4B_EINVAL, "q4_0 GEMM: bad grouped-mode arguments");
-  const bool aligned = g.W.nb % 2 == 0 && d.W.nb % 2 == 0;
+  const bool ga = g.W.nb % 2 == 0, da = d.W.nb % 2 == 0;
   if (g.epi == GEMM_GLU) {
-    if (!aligned) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d blocks", g.W.nb);
-    gemm::go_grp<GEMM_GLU, true>(g, d, st);
-  } else if (aligned) {
-    gemm::go_grp<GEMM_F32, true>(g, d, st);
+    if (!ga || !da) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d blocks", g.W.nb);
+    gemm::go_grp<GEMM_GLU, true, true>(g, d, st);
   } else {
-    gemm::go_grp<GEMM_F32, false>(g, d, st);
+    (ga ? da ? gemm::go_grp<GEMM_F32, true, true> : gemm::go_grp<GEMM_F32, true, false>
+        : da ? gemm::go_grp<GEMM_F32, false, true> : gemm::go_grp<GEMM_F32, false, false>)(g, d, st);
   }
   E4B_HIP(hipGetLastError());
   return E4B_OK;
