@@ -110,9 +110,10 @@ struct Shape {
 
 // EPI GEMM_GLU: NT = 2, tile 0 a gate tile, tile 1 the up tile of the same
 // outputs.  Other epilogues: NT tiles of 32 adjacent row groups.
-// (bx, by): row tile and token tile; bufa, bufb: two separate LDS arrays of
-// Shape::BUF pieces (the compiler then knows that the copies into one do not
-// alias the reads of the other), scb: the scales of two stages.
+// bx: row tile; by: first token row (GRP: entry of the tile table); bufa,
+// bufb: two separate LDS arrays of Shape::BUF pieces (the compiler then knows
+// that the copies into one do not alias the reads of the other), scb: the
+// scales of two stages.
 template <int T, int NT, int RW, int KW, int KBL, int EPI, bool GRP, bool ALN>
 DEV void gemm_tile(const GemmArgs& a, int nb, int nbs, int bx, int by, u32x4* bufa, u32x4* bufb, uint32_t* scb) {
   using S = Shape<T, NT, RW, KW, KBL>;
@@ -136,7 +137,7 @@ DEV void gemm_tile(const GemmArgs& a, int nb, int nbs, int bx, int by, u32x4* bu
     tok0 = tl.y;
     nrows = tl.z;
   } else {
-    tok0 = by * TOK;
+    tok0 = by;
     nrows = min(TOK, a.M - tok0);
   }
   const int64_t c0 = (int64_t)bx * UC;
@@ -415,30 +416,36 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_q40_gemm(GemmArgs a, int nb
   __shared__ __align__(16) u32x4 bufa[S::BUF];
   __shared__ __align__(16) u32x4 bufb[S::BUF];
   __shared__ __align__(16) uint32_t scb[ALN ? S::COLS * S::SB : 4];
-  gemm_tile<T, NT, RW, KW, KBL, EPI, false, ALN>(a, nb, nbs, blockIdx.x, blockIdx.y, bufa, bufb, scb);
+  gemm_tile<T, NT, RW, KW, KBL, EPI, false, ALN>(a, nb, nbs, blockIdx.x, blockIdx.y * S::TOK, bufa, bufb, scb);
 }
 
 // A grouped product and an ordinary one in one launch: the first ndense
-// workgroups are tiles of d (dbx of them side by side), the rest of g.  The dense branch of an MoE layer alone leaves most of the
+// workgroups are tiles of d (dbx of them side by side, dtok token rows each),
+// the rest of g.  The dense branch of an MoE layer alone leaves most of the
 // chip idle; in front of the experts' tiles it fills the workgroup slots that
 // their last, part-empty wave leaves: a half-layer over 512 tokens 247 -> 239
 // us (MI355X; the dense branch in launches of its own: 30 + 17 us).
 //
-// An expert's last rows often fit one token tile: half the work of two.
+// Tiles of at most 32 live rows (an expert's last draws, the dense branch's
+// few or last tokens) are one token tile a wave, half the work of two; K is
+// summed in the same order, so a token's result does not depend on its tile.
 // GALN, DALN: whether g's and d's rows have an even number of blocks, each for
 // its own tiles: a dense width of an odd number must not put the experts'
 // product, the far larger one, on the kernel that loads scales singly.
 template <int T, int NT, int RW, int KW, int KBL, int EPI, bool GALN, bool DALN>
 __global__ __launch_bounds__(64 * RW * KW, 2) void k_q40_gemm_grp(GemmArgs g, GemmArgs d, int ndense, int dbx,
-                                                                  int gbx) {
+                                                                  int dtok, int gbx) {
   using S = Shape<T, NT, RW, KW, KBL>;
   __shared__ __align__(16) u32x4 bufa[S::BUF];
   __shared__ __align__(16) u32x4 bufb[S::BUF];
   __shared__ __align__(16) uint32_t scb[GALN || DALN ? S::COLS * S::SB : 4];
   int id = blockIdx.x;
   if (id < ndense) {
-    const int by = id / dbx, bx = id % dbx;
-    gemm_tile<T, NT, RW, KW, KBL, EPI, false, DALN>(d, d.W.nb, d.W.nb, bx, by, bufa, bufb, scb);
+    const int tok0 = id / dbx * dtok, bx = id % dbx;
+    if (T == 2 && (dtok <= 32 || d.M - tok0 <= 32))
+      gemm_tile<1, NT, RW, KW, KBL, EPI, false, DALN>(d, d.W.nb, d.W.nb, bx, tok0, bufa, bufb, scb);
+    else
+      gemm_tile<T, NT, RW, KW, KBL, EPI, false, DALN>(d, d.W.nb, d.W.nb, bx, tok0, bufa, bufb, scb);
     return;
   }
   id -= ndense;

@@ -16,9 +16,16 @@ void go_grp(const GemmArgs& g, const GemmArgs& d, hipStream_t st) {
   static_assert(TOK == kGroupTileRows, "a group's row tile");
   const int64_t gu = EPI == GEMM_GLU ? g.ff : g.group_rows, du = EPI == GEMM_GLU ? d.ff : d.W.rows;
   const int gbx = (int)((gu + UC - 1) / UC), dbx = (int)((du + UC - 1) / UC);
-  const int ndense = dbx * ((d.M + TOK - 1) / TOK);
+  // Up to 64 tokens the dense product's serial K loop can outlast the experts'
+  // tiles, and in tiles of 32 tokens a stage of it takes 3/4 of the time.  A
+  // half-layer of 1 token 57 -> 48 us (hidden 2816, 128 experts of 704, dense
+  // 2112), of 37 tokens 49 -> 42 (hidden 1024, 16 experts of 160, dense 2112),
+  // where launches of its own took 56 and 45.  At 128 tokens tiles of 32 were
+  // 10 % faster at the second shape and 2 % slower at the first with dense 2080.
+  const int dtok = d.M <= 64 ? 32 : TOK;
+  const int ndense = dbx * ((d.M + dtok - 1) / dtok);
   hipLaunchKernelGGL((k_q40_gemm_grp<T, NT, RW, KW, KBL, EPI, GALN, DALN>), dim3((unsigned)(ndense + gbx * g.max_tiles)),
-                     dim3(64 * RW * KW), 0, st, g, d, ndense, dbx, gbx);
+                     dim3(64 * RW * KW), 0, st, g, d, ndense, dbx, dtok, gbx);
 }
 
 }  // namespace gemm
