@@ -128,13 +128,16 @@ int e4b_k_q40_gemv_geglu(const void* w_packed, int64_t ff, int64_t cols, const v
  * GEMV (replaces the multi-column GEMVs of the reference's prefill,
  * kernels/q40mm.wgsl and kernels/q40sg.wgsl driven by
  * src/engine-a4b.js:465-585): x is f16[m][cols] row-major (m tokens),
- * y is f32[m][rows] row-major, y[t][r] = W[r] . x[t].  cols % 32 == 0. */
+ * y is f32[m][rows] row-major, y[t][r] = W[r] . x[t].  cols % 32 == 0.
+ * The products are exact and the order of their f32 sums follows from rows,
+ * cols and m: the same call gives the same bits, calls of another m may differ
+ * in a row's last ones. */
 int e4b_k_q40_gemm(const void* w_packed, int64_t rows, int64_t cols, const void* x_f16, int m, float* y,
                    void* stream);
 
 /* Batched gate/up + GeGLU: w_packed is [2*ff][cols] (gate rows then up
  * rows), x f16[m][cols], out f16[m][ff] = f16(gelu_tanh(gate) * up)
- * (kernels/q40gu.wgsl:62-119 per token). */
+ * (kernels/q40gu.wgsl:62-119 per token); the sums' order as there. */
 int e4b_k_q40_gemm_geglu(const void* w_packed, int64_t ff, int64_t cols, const void* x_f16, int m, void* out_f16,
                          void* stream);
 
@@ -250,7 +253,8 @@ int e4b_k_moe_layer(const e4b_moe_weights* w, const float* h, float* h_out, uint
  * the m*8 expert draws are sorted by expert and each expert's weight rows
  * are read once per tile of up to 64 draws (MFMA GEMMs).  h, h_out
  * f32[m][hidden]; topk_idx u32[m][8], topk_w f32[m][8], dense_out /
- * moe_out f32[m][hidden] may be NULL.  1 <= m <= 1024. */
+ * moe_out f32[m][hidden] may be NULL.  1 <= m <= 1024.  A row's results do
+ * not depend on m or on the other rows. */
 int e4b_k_moe_prefill(const e4b_moe_weights* w, const float* h, int m, float* h_out, uint32_t* topk_idx,
                       float* topk_w, float* dense_out, float* moe_out, void* stream);
 
@@ -365,8 +369,11 @@ int  e4b_step(e4b_ctx* ctx, uint32_t token, uint32_t pos, float* logits_or_null,
  * expert-grouped GEMMs, src/engine-a4b.js:478-549); the lm-head runs once,
  * for the last token.  argmax_out = greedy
  * continuation of the last prompt token, which is also fed back as the next
- * e4b_decode input.  E4B_FLAG_STEP_PREFILL runs the prompt through the decode
- * step instead. */
+ * e4b_decode input.  The order of the f32 sums follows from a chunk's length:
+ * the same prompt gives the same bits again, while the K/V rows that it shares
+ * with a longer or shorter prompt may differ in rounding.
+ * E4B_FLAG_STEP_PREFILL runs the prompt through the decode step instead, where
+ * a row depends on nothing behind it. */
 int  e4b_prefill(e4b_ctx* ctx, const uint32_t* ids, uint32_t n, uint32_t* argmax_out);
 /* the prompt token by token through the decode step (the prompt loop of
  * generateFast, src/engine-a4b.js:826-829: step(t, pos) per prompt token,
