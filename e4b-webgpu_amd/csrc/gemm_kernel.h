@@ -22,11 +22,12 @@
 //
 // What bounds it: per 32 x 32 tile and block, two matrix instructions (64
 // cycles of a SIMD's matrix core) and 16 scale multiply-adds plus the nibble
-// conversion (9 instructions a row tile, shared by the T token tiles) on the
-// vector unit, 4 cycles each.  The two units run side by side only if the
-// instructions are interleaved: a register-only loop of the pair takes 34.5
-// ns (matrix alone), 34.9 ns (multiply-adds alone), 47.5 ns (both, two waves
-// per SIMD, 1.9 GHz), i.e. 1.4 PFLOP/s, while this card's library f16 product
+// conversion (9 instructions a nibble word, two words a lane and row tile,
+// shared by the T token tiles) on the vector unit, 4 cycles each.  The two
+// units run side by side only if the instructions are interleaved: a
+// register-only loop takes 32.6 ns a tile and SIMD with the matrix
+// instructions alone, 37.3 with the multiply-adds alone, 43.6 with both (two
+// waves per SIMD), i.e. 1.5 PFLOP/s, while this card's library f16 product
 // reaches 1.1-1.2.  So the loop below is written as a software pipeline
 // (multiply-adds of one tile between the matrix instructions of the next).
 //
@@ -34,7 +35,7 @@
 // that share the K loop (each takes KBL of every KW KBL blocks; their sums
 // meet in LDS at the end).  Splitting K inside the workgroup instead of over
 // the grid needs no partial sums in memory, so also a call that has no
-// scratch can fill the chip: a 2048 x 16384 matrix over 512 tokens 148 -> 59
+// scratch can fill the chip: a 2048 x 16384 matrix over 512 tokens 148 -> 55
 // us, 3072 x 2048 over 37 tokens 17.7 -> 5 us (MI355X; before: 4 waves, one
 // K group, operands staged through registers).
 #pragma once

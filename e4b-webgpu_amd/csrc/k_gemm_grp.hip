@@ -49,7 +49,8 @@ int launch_q40_gemm_grouped(const GemmArgs& g, const GemmArgs& d, hipStream_t st
     return e4b_fail(E4B_EINVAL, "q4_0 GEMM: bad grouped-mode arguments");
   const bool ga = g.W.nb % 2 == 0, da = d.W.nb % 2 == 0;
   if (g.epi == GEMM_GLU) {
-    if (!ga || !da) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d blocks", g.W.nb);
+    if (!ga || !da) return e4b_fail(E4B_EINVAL, "q4_0 GEMM: no grouped GeGLU over rows of %d and %d blocks", g.W.nb,
+                               d.W.nb);
     gemm::go_grp<GEMM_GLU, true, true>(g, d, st);
   } else {
     (ga ? da ? gemm::go_grp<GEMM_F32, true, true> : gemm::go_grp<GEMM_F32, true, false>

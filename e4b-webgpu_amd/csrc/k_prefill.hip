@@ -299,12 +299,16 @@ __global__ __launch_bounds__(64) void k_headprep_rows(const float* __restrict__ 
 // rows of a fragment share their banks), and V^T is read with the transposing
 // ds_read_b64_tr_b16: a group of 16 lanes reads 4 keys x 16 dims, lane i
 // addressing key i / 4, dims 4 (i % 4), and receives dim i of the 4 keys.
-// Per call with its merge of the splits, before -> now: 512 queries x 8 heads
-// over a window of 512 keys 31.2 -> 25.7 us, at the end of 4096 keys 86.9 ->
-// 60 us, 512 x 16 heads over 8 KV heads 43.3 -> 33.9 us, one query over 3001
-// keys 37.6 -> 25.7 us.  Tried and left out, all at the same time or slower:
-// more of a tile's fragments read ahead into registers, four tiles in flight
-// with one workgroup per CU (29.9 us), the loop unrolled over both buffers.
+// Per call with its merge of the splits, 40 calls back to back, before -> now:
+// 512 queries x 8 heads over a window of 512 keys 31.1 -> 25.7 us, at the end
+// of 4096 keys 84 -> 55 us, 512 x 16 heads over 8 KV heads 42.6 -> 33.2 us,
+// one query over 3001 keys 37.6 -> 25.8 us.  Head dim 512 (this kernel alone,
+// 512 queries x 16 heads over 2 KV heads; 96 KB of LDS, so one workgroup a CU
+// where two fitted before): the first 512 positions 72 -> 53 us, the second to
+// fourth 216 -> 170, 33 queries 14.5 -> 9.9 us.  Tried and left out, all at the
+// same time or slower (the first call): more of a tile's fragments read ahead
+// into registers, four tiles in flight with one workgroup per CU (29.9 us),
+// the loop unrolled over both buffers.
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef __fp16 tr4 __attribute__((__vector_size__(8)));

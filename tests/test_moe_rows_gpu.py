@@ -1,5 +1,5 @@
 """The MoE half-layer over token rows at the edges of its kernels: row counts
-around the router's 8 rows a block and the grouped product's 64-row tiles,
+around the router's 2 rows a block and the grouped product's 64-row tiles,
 expert counts around its 16 experts a block, hidden sizes from one piece of a
 row to all twelve, odd block counts in either down projection, and draws that
 all go to the same 8 experts.
