@@ -1,7 +1,7 @@
 """ctypes wrapper of the CPU oracle (oracle/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and the
-cpu_baseline leg of bench.py, and only as the checker / CPU baseline.  The
+cpu_baseline leg of bench.py, and only as the reference result / CPU baseline.  The
 product library never loads it.
 
 Parity status of each restated function (how it is pinned) is listed in

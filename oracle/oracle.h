@@ -4,7 +4,7 @@
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product (the HIP library under
  * e4b-webgpu_amd/) links, loads or calls this code.  Only tests/, the smoke()
  * entry of __graft_entry__.py and the cpu_baseline leg of bench.py use it, and
- * only as the checker (or as the timed CPU baseline), never as the thing that
+ * only as the reference result (or as the timed CPU baseline), never as the thing that
  * is measured or shipped.
  *
  * Every function restates one piece of the reference's WGSL/JS semantics and

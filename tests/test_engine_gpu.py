@@ -1,6 +1,6 @@
 """End-to-end parity of the decode engine (libe4b, HIP) with the CPU oracle.
 
-Tolerances (stated, as the north star asks):
+Tolerances:
   * greedy tokens: bit-exact, except at a near-tie where the oracle's top-2
     logit margin is below 2e-3 of its logit range (reported, then the oracle's
     choice is fed to both sides so the comparison continues in lock-step);
@@ -207,7 +207,7 @@ def test_c4_full_model_lockstep():
 
 @pytest.mark.slow
 def test_c4_greedy_256_steps():
-    # the north-star bar: the GPU-fed greedy sequence at the E4B shape equals
+    # the GPU-fed greedy sequence at the E4B shape equals
     # the oracle's over 256 decode steps (near-ties reported, none expected)
     cfg = E4BConfig(max_seq=1024)
     eng, om = build(cfg, 3)
